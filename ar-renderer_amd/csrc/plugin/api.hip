@@ -21,6 +21,12 @@
 #include "sheen_table.h"
 #include "trace_dev.h"
 
+// The traversal kernels' register budget (see pt.hip, PG_WAVES).
+#ifndef PG_TRACE_WAVES
+#define PG_TRACE_WAVES 8
+#endif
+#define PG_TRACE_WAVES_ATTR __attribute__((amdgpu_waves_per_eu(PG_TRACE_WAVES, 8)))
+
 namespace pgpu {
 
 namespace {
@@ -39,12 +45,13 @@ bool gEnumerated = false;
 
 // Scratch of the allocation-free ray query (prgpu_trace_rays_noalloc), one copy per GPU, held
 // until the process ends. Words [0, kScratchHeadWords) hold the traversal stack-overflow flag
-// (word 0); the rest holds the per-lane spill slabs of the traversal stacks. Host code never
+// (word 0) and the ray counters (from word kFeedStride on); the rest holds the per-lane spill slabs of the traversal stacks. Host code never
 // passes `scratch` itself to a kernel: it uses the device address that hipGetSymbolAddress
 // returns for the current device (Device::scratch).
 constexpr size_t kScratchBytes = size_t(64) << 20;
 constexpr size_t kScratchWords = kScratchBytes / sizeof(uint32_t);
-constexpr size_t kScratchHeadWords = 64;  // 256 B, so the spill slabs start 256-B aligned
+constexpr size_t kScratchHeadWords = 1024;  // a multiple of 256 B, so the spill slabs start 256-B aligned
+static_assert(kFeedStride + kFeedInts <= int(kScratchHeadWords), "ray counters exceed the scratch head");
 static __device__ __align__(256) uint32_t scratch[kScratchWords];
 
 void SetErr(char *err, int len, const std::string &m) {
@@ -175,8 +182,8 @@ Device &Get(int index) {
         hipDeviceProp_t prop;
         PG_CHECK(hipGetDeviceProperties(&prop, d.id));
         d.cus = prop.multiProcessorCount;
-        d.flags.ensure(64);
-        PG_CHECK(hipMemset(d.flags.p, 0, 64));
+        d.flags.ensure(kScratchHeadWords * sizeof(uint32_t));
+        PG_CHECK(hipMemset(d.flags.p, 0, kScratchHeadWords * sizeof(uint32_t)));
         // Device address of this GPU's copy of the allocation-free query's scratch array.
         void *sp = nullptr;
         PG_CHECK(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
@@ -186,40 +193,58 @@ Device &Get(int index) {
 }
 
 __global__ void k_scratch_clear(uint32_t *words, int n) {
-    const int i = int(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i < n) words[i] = 0u;
+    for (int i = int(threadIdx.x); i < n; i += int(blockDim.x)) words[i] = 0u;
 }
 
 
 // With kStats (profile mode 2) every lane adds its rays, nodes fetched and leaf records tested
-// to counters[0..2] (closest hit) or counters[3..5] (any hit).
+// to counters[0..2] (closest hit) or counters[3..5] (any hit). The fetch counters start at zero.
 template <bool kStats>
-__global__ __launch_bounds__(kTraceBlock) void k_trace_rays(TraceCtx c, const prgpu::RayEx *rays, prgpu::HitEx *hits,
-                                                            int64_t n, int anyHit, unsigned long long *counters) {
+__global__ __launch_bounds__(kTraceBlock) PG_TRACE_WAVES_ATTR void k_trace_rays(
+    TraceCtx c, const prgpu::RayEx *rays, prgpu::HitEx *hits, int n, int anyHit, int *fetch, unsigned long long *counters) {
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
-    const int64_t stride = int64_t(gridDim.x) * blockDim.x;
     TraceStats st;
     unsigned long long traced = 0;
-    for (int64_t i = tid; i < n; i += stride) {
-        const prgpu::RayEx rr = rays[i];
-        DRay r{rr.o.x, rr.o.y, rr.o.z, rr.d.x, rr.d.y, rr.d.z};
-        DHit h;
-        bool hit = anyHit ? dev_trace<true, kStats>(c, r, rr.tMax, &h, lds, tid, &st)
-                          : dev_trace<false, kStats>(c, r, rr.tMax, &h, lds, tid, &st);
-        prgpu::HitEx o;
-        o.t = hit ? h.t : 0.f;
-        o.prim = hit ? h.prim : -1;
-        o.b1 = hit ? h.b1 : 0.f;
-        o.b2 = hit ? h.b2 : 0.f;
-        hits[i] = o;
-        ++traced;
-    }
+    trace_queue<kStats>(
+        c, n, fetch, lds, tid, &st,
+        [&](int i, DRay &r, TravState &t) {
+            const prgpu::RayEx rr = rays[i];
+            r = DRay{rr.o.x, rr.o.y, rr.o.z, rr.d.x, rr.d.y, rr.d.z};
+            trace_begin(t, r, rr.tMax, anyHit != 0);
+        },
+        [&](int i, DRay &, TravState &t) {
+            prgpu::HitEx o;
+            o.t = t.found() ? t.tMax : 0.f;
+            o.prim = t.prim;
+            o.b1 = t.b1;
+            o.b2 = t.b2;
+            hits[i] = o;
+            ++traced;
+            return false;
+        });
     if (kStats && traced) {
         unsigned long long *ctr = counters + (anyHit ? 3 : 0);
         atomicAdd(&ctr[0], traced);
-        atomicAdd(&ctr[1], (unsigned long long)st.nodes);
-        atomicAdd(&ctr[2], (unsigned long long)st.recs);
+        atomicAdd(&ctr[1], (unsigned long long)(anyHit ? st.anyNodes : st.nodes));
+        atomicAdd(&ctr[2], (unsigned long long)(anyHit ? st.anyRecs : st.recs));
+    }
+}
+
+// Traces n device rays in launches of at most kMaxLaunchRays. words: [0] the stack overflow flag
+// (c.errorFlag, cleared here when clearFlag is set), from kFeedStride on the launches' ray counters.
+constexpr int kAnyGrid = 0x7fffffff;
+constexpr int64_t kMaxLaunchRays = int64_t(1) << 30;
+void LaunchTraceRays(Device &d, const TraceCtx &c, uint32_t *words, bool clearFlag, int maxGrid, const prgpu::RayEx *rays,
+                     int64_t n, int anyHit, prgpu::HitEx *hits, unsigned long long *counters) {
+    for (int64_t at = 0; at < n; at += kMaxLaunchRays) {
+        const int m = int(std::min(n - at, kMaxLaunchRays));
+        const bool flag = clearFlag && at == 0;
+        hipLaunchKernelGGL(k_scratch_clear, dim3(1), dim3(kTraceBlock), 0, d.stream, flag ? words : words + kFeedStride,
+                           kFeedInts + (flag ? kFeedStride : 0));
+        auto *k = counters ? k_trace_rays<true> : k_trace_rays<false>;
+        hipLaunchKernelGGL(k, dim3(std::min(TraceGrid(d, m), maxGrid)), dim3(kTraceBlock), 0, d.stream, c, rays + at, hits + at,
+                           m, anyHit, reinterpret_cast<int *>(words + kFeedStride), counters);
     }
 }
 
@@ -250,13 +275,8 @@ void EnsureGeometry(Device &d, const prgpu::Primitive *prims, int count) {
     if (key == d.geomKey && d.nodes.p) return;
     WideBVH bvh;
     BuildWideBVH(prims, count, &bvh);
-    if (bvh.nodes.empty()) {  // empty scene: a root with no children
-        bvh.nodes.emplace_back();
-        std::memset(&bvh.nodes[0], 0, sizeof(WNode));
-        bvh.depth = 1;
-    }
     d.nodes.upload(bvh.nodes.data(), bvh.nodes.size(), d.stream);
-    d.recs.upload(bvh.recs.data(), bvh.recs.size(), d.stream);  // an empty scene gets a small unread buffer
+    d.recs.upload(bvh.recs.data(), bvh.recs.size(), d.stream);
     d.depth = bvh.depth;
     d.nodeCount = int(bvh.nodes.size());
     d.recCount = int(bvh.recs.size());
@@ -285,7 +305,10 @@ TraceCtx MakeTraceCtx(Device &d) {
 }
 
 int TraceGrid(const Device &d, int64_t n) {
-    int64_t blocks = (n + kTraceBlock - 1) / kTraceBlock;
+    // A short queue is spread over kSpreadWaves waves (see trace_dev.h, RayFeed), down to one ray each.
+    constexpr int64_t kWaves = kTraceBlock / 64;
+    const int64_t spread = std::min<int64_t>((n + kWaves - 1) / kWaves, kSpreadWaves / kWaves);
+    const int64_t blocks = std::max((n + kTraceBlock - 1) / kTraceBlock, spread);
     const int perCU = std::max(1, std::min(d.tune.traceBlocksPerCU, kTraceBlocksPerCU));
     return int(std::max<int64_t>(1, std::min<int64_t>(blocks, int64_t(d.cus) * perCU)));
 }
@@ -361,14 +384,9 @@ PRGPU_API int prgpu_trace_rays(int deviceIndex, const prgpu::SceneDescEx *sd, co
         if (n == 0) return 0;
         d.rays.upload(rays, size_t(n), d.stream);
         d.hits.ensure(size_t(n) * sizeof(prgpu::HitEx));
-        if (d.profileMode >= 2 && d.travCounters.p)
-            hipLaunchKernelGGL(k_trace_rays<true>, dim3(TraceGrid(d, n)), dim3(kTraceBlock), 0, d.stream,
-                               MakeTraceCtx(d), d.rays.as<prgpu::RayEx>(), d.hits.as<prgpu::HitEx>(), n, anyHit,
-                               d.travCounters.as<unsigned long long>());
-        else
-            hipLaunchKernelGGL(k_trace_rays<false>, dim3(TraceGrid(d, n)), dim3(kTraceBlock), 0, d.stream,
-                               MakeTraceCtx(d), d.rays.as<prgpu::RayEx>(), d.hits.as<prgpu::HitEx>(), n, anyHit,
-                               static_cast<unsigned long long *>(nullptr));
+        LaunchTraceRays(d, MakeTraceCtx(d), d.flags.as<uint32_t>(), false, kAnyGrid, d.rays.as<prgpu::RayEx>(), n, anyHit,
+                        d.hits.as<prgpu::HitEx>(),
+                        d.profileMode >= 2 && d.travCounters.p ? d.travCounters.as<unsigned long long>() : nullptr);
         PG_CHECK(hipGetLastError());
         PG_CHECK(hipMemcpyAsync(hits, d.hits.p, size_t(n) * sizeof(prgpu::HitEx), hipMemcpyDeviceToHost, d.stream));
         CheckTraceFlags(d);
@@ -435,9 +453,7 @@ PRGPU_API int prgpu_trace_rays_noalloc(int deviceIndex, const prgpu::SceneDescEx
         c.spillStride = grid * kTraceBlock;
         c.errorFlag = reinterpret_cast<int *>(d.scratch);
         // The scratch keeps the previous call's contents: the overflow flag must start at zero.
-        hipLaunchKernelGGL(k_scratch_clear, dim3(1), dim3(64), 0, d.stream, d.scratch, 1);
-        hipLaunchKernelGGL(k_trace_rays<false>, dim3(grid), dim3(kTraceBlock), 0, d.stream, c, rays, hits, n, anyHit,
-                           static_cast<unsigned long long *>(nullptr));
+        LaunchTraceRays(d, c, d.scratch, true, grid, rays, n, anyHit, hits, nullptr);
         PG_CHECK(hipGetLastError());
         int f = 0;
         PG_CHECK(hipMemcpyAsync(&f, d.scratch, sizeof(int), hipMemcpyDeviceToHost, d.stream));

@@ -207,9 +207,9 @@ Box3 PrimBounds(const prgpu::Primitive &p) {
 #endif
 constexpr int kSurfaceWaves = PG_SURFACE_WAVES, kMaterialWaves = PG_MATERIAL_WAVES;
 
-// Bufs::counts: queue lengths and the ray fetch counters of the persistent traversals.
-constexpr int kFetchIntersect = 16, kFetchShadow = 32, kCountsInts = 48, kCountsBytes = kCountsInts * 4;
-static_assert(kFetchParts <= 16, "fetch counters overlap");
+// Bufs::counts: queue lengths (in one line) and the ray counters of the persistent traversals.
+constexpr int kFetchIntersect = 32, kFetchShadow = kFetchIntersect + kFeedInts, kCountsInts = kFetchShadow + kFeedInts,
+              kCountsBytes = kCountsInts * 4;
 
 struct PTScene {
     DevBuf prims, mats, specs, knots, lights, lightArea, lnodes, leafOf, infinite, powerCdf, powerFunc, media, grid, sheen;
@@ -716,8 +716,7 @@ struct Bufs {
                   // shadow rays are traced with the next bounce's closest hits), [3..5] plain
                   // material queues, [6] medium scattering vertices, [9] emission queue, [10]
                   // coated / sheen material queue,
-                  // [16..16+P) closest-hit fetch counters, [32..32+P) shadow fetch counters
-                  // (P = kFetchParts)
+                  // then the ray counters of the traversal and of the shadow walk (kFeedInts each)
     float2 *pfilm;
     float4 *xyz;
     // shadow records, one per path slot (a path makes at most one shadow ray per bounce)
@@ -928,40 +927,34 @@ __global__ __launch_bounds__(kBlock) void k_camera(const DevScene *__restrict__ 
         for (int j = 0; j < kGuideRecords; ++j) b.trec[6 * j * size_t(b.qcap) + slot] = make_float4(0, 0, 0, 0);
 }
 
-// Closest hits of the queued paths. Persistent: each lane takes a new ray from the queue front as
-// soon as its previous one completes (fetch_rays_parts), so a wave's lanes stay busy while ray
-// lengths differ and the rays in flight stay a narrow, coherent part of the queue.
+// A closest hit as the path state holds it: distance, primitive (-1: a miss), barycentrics.
+__device__ __forceinline__ float4 closest_hit(const TravState &t) {
+    return t.found() ? make_float4(t.tMax, __int_as_float(t.prim), t.b1, t.b2) : make_float4(0, __int_as_float(-1), 0, 0);
+}
+
+// Closest hits of the queued paths (persistent, see trace_queue).
 template <bool kStats>
 __global__ __launch_bounds__(kTraceBlock) PG_WAVES(8) void k_intersect(const DevScene *__restrict__ sp, Bufs b, const int *queue,
                                                            const int *count, int *fetch, unsigned long long *counters) {
     const DevScene &s = *sp;
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
-    const int n = *count;
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
     TraceStats st;
     uint32_t rays = 0;
-    int idx = -1, slot = 0;
-    bool started = false;
-    DRay r{};
-    TravState t{};
-    FetchState fs = fetch_begin();
-    while (fetch_rays_parts(fetch, n, idx, fs)) {
-        if (idx >= 0 && !started) {
-            slot = queue[idx];
-            float4 o = b.o[slot], d = b.d[slot];
+    int slot = 0;
+    trace_queue<kStats>(
+        s.trace, *count, fetch, lds, tid, &st,
+        [&](int i, DRay &r, TravState &t) {
+            slot = queue[i];
+            const float4 o = b.o[slot], d = b.d[slot];
             r = DRay{o.x, o.y, o.z, d.x, d.y, d.z};
-            trace_begin(t, r, kInfF);
-            started = true;
-        }
-        if (!trace_turn(idx >= 0, t.cur)) continue;
-        if (trace_step<false, kStats>(s.trace, r, t, lds, tid, &st)) {
-            b.hit[slot] = t.found ? make_float4(t.hit.t, __int_as_float(t.hit.prim), t.hit.b1, t.hit.b2)
-                                  : make_float4(0, __int_as_float(-1), 0, 0);
+            trace_begin(t, r, kInfF, false);
+        },
+        [&](int, DRay &, TravState &t) {
+            b.hit[slot] = closest_hit(t);
             ++rays;
-            idx = -1;
-            started = false;
-        }
-    }
+            return false;
+        });
     if (kStats && rays) {
         atomicAdd(&counters[0], (unsigned long long)rays);
         atomicAdd(&counters[1], (unsigned long long)st.nodes);
@@ -1709,13 +1702,9 @@ __device__ __forceinline__ void shadow_add(const Bufs &b, int slot, const SS &T,
 // previous bounce (scenes without media or interfaces, where a shadow ray is one any-hit query).
 // The two are independent: a shadow ray only adds to its path's radiance, which this bounce's
 // surface and emission stages read after the launch, so contributions are added in the same order
-// as with a launch of their own and every sample's result is unchanged. A wave takes closest rays
-// until that queue is drained, then shadow rays, so a bounce has one traversal tail instead of
-// two; late bounces, where a few thousand rays take the whole launch latency, cost half as much.
-#ifndef PG_FUSED_SHADOW
-#define PG_FUSED_SHADOW 1
-#endif
-constexpr bool kFusedShadow = PG_FUSED_SHADOW != 0;
+// as with a launch of their own and every sample's result is unchanged. The shadow rays follow the
+// closest rays in one run of items, so a bounce has one traversal tail instead of two; late bounces,
+// where a few thousand rays take the whole launch latency, cost half as much.
 constexpr int kShadowCountB = 11;  // the second shadow queue length (see Bufs::counts)
 __host__ __device__ constexpr int shadow_count_index(int curIdx) { return curIdx ? kShadowCountB : 2; }
 
@@ -1723,182 +1712,105 @@ template <bool kStats>
 __global__ __launch_bounds__(kTraceBlock) PG_WAVES(8) void k_trace_bounce(const DevScene *__restrict__ sp, Bufs b,
                                                                         const int *queue, const int *count,
                                                                         const int *shadowCount, int *fetch,
-                                                                        int *shadowFetch, unsigned long long *counters) {
+                                                                        unsigned long long *counters) {
     const DevScene &s = *sp;
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
     const int n = *count, ns = *shadowCount;
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
-    TraceStats stc, sts;
+    TraceStats st;
     uint32_t raysC = 0, raysS = 0;
-    int idx = -1, slot = 0;
-    bool shadow = false, started = false;
-    DRay r{};
-    TravState t{};
-    FetchState fc = fetch_begin(), fs = fetch_begin();
-    while (true) {
-        bool more;
-        if (!fc.done) {
-            const bool idle = idx < 0;
-            more = fetch_rays_parts(fetch, n, idx, fc);
-            if (idle && idx >= 0) shadow = false;
-        }
-        if (fc.done) {
-            const bool idle = idx < 0;
-            more = fetch_rays_parts(shadowFetch, ns, idx, fs);
-            if (idle && idx >= 0) shadow = true;
-        }
-        if (!more) break;
-        if (idx >= 0 && !started) {
-            if (shadow) {
-                slot = b.sq[idx];
-                const float4 so = b.so[slot], sd = b.sd[slot];
-                r = DRay{so.x, so.y, so.z, sd.x, sd.y, sd.z};
-                trace_begin(t, r, kShadowTMax);
-                t.any = true;
-            } else {
-                slot = queue[idx];
-                const float4 o = b.o[slot], d = b.d[slot];
-                r = DRay{o.x, o.y, o.z, d.x, d.y, d.z};
-                trace_begin(t, r, kInfF);
-            }
-            started = true;
-        }
-        if (!trace_turn(idx >= 0, t.cur)) continue;
-        TraceStats one;
-        const bool fin = trace_step<false, kStats, true>(s.trace, r, t, lds, tid, &one);
-        if (kStats) {
-            sts.nodes += shadow ? one.nodes : 0u;
-            sts.recs += shadow ? one.recs : 0u;
-            stc.nodes += shadow ? 0u : one.nodes;
-            stc.recs += shadow ? 0u : one.recs;
-        }
-        if (fin) {
-            if (shadow) {
+    int slot = 0;
+    trace_queue<kStats>(
+        s.trace, n + ns, fetch, lds, tid, &st,
+        [&](int i, DRay &r, TravState &t) {
+            const bool shadow = i >= n;
+            slot = shadow ? b.sq[i - n] : queue[i];
+            const float4 o = (shadow ? b.so : b.o)[slot], d = (shadow ? b.sd : b.d)[slot];
+            r = DRay{o.x, o.y, o.z, d.x, d.y, d.z};
+            trace_begin(t, r, shadow ? kShadowTMax : kInfF, shadow);
+        },
+        [&](int, DRay &, TravState &t) {
+            if (t.any) {
                 ++raysS;
-                if (!t.found) {
+                if (!t.found()) {
                     const float4 spk = b.sp[slot], snk = b.sn[slot];
                     shadow_add(b, slot, SS(1.f), spk.w, snk.w);
                 }
             } else {
                 ++raysC;
-                b.hit[slot] = t.found ? make_float4(t.hit.t, __int_as_float(t.hit.prim), t.hit.b1, t.hit.b2)
-                                      : make_float4(0, __int_as_float(-1), 0, 0);
+                b.hit[slot] = closest_hit(t);
             }
-            idx = -1;
-            started = false;
-        }
-    }
+            return false;
+        });
     if (kStats && (raysC || raysS)) {
         atomicAdd(&counters[0], (unsigned long long)raysC);
-        atomicAdd(&counters[1], (unsigned long long)stc.nodes);
-        atomicAdd(&counters[2], (unsigned long long)stc.recs);
+        atomicAdd(&counters[1], (unsigned long long)st.nodes);
+        atomicAdd(&counters[2], (unsigned long long)st.recs);
         atomicAdd(&counters[3], (unsigned long long)raysS);
-        atomicAdd(&counters[4], (unsigned long long)sts.nodes);
-        atomicAdd(&counters[5], (unsigned long long)sts.recs);
+        atomicAdd(&counters[4], (unsigned long long)st.anyNodes);
+        atomicAdd(&counters[5], (unsigned long long)st.anyRecs);
     }
 }
 
-// Transmittance of the shadow records (src/scene/scene.cpp:41-59) and the deferred add().
-// Without media or interfaces a shadow ray is one any-hit query, traversed persistently as in
-// k_intersect; otherwise each ray walks its interface crossings to completion.
-// Transmittance of one shadow record (src/scene/scene.cpp:41-59): one any-hit query, or with
-// interfaces a walk through their crossings, with the media's transmittance along the way; then
-// the deferred add().
-template <bool kMedia, bool kInterfaces, bool kStats>
-__device__ __forceinline__ void shadow_walk(const DevScene &s, const Bufs &b, int slot, uint32_t *lds, int tid,
-                                            TraceStats *ts) {
-    float4 so = b.so[slot], sd = b.sd[slot], spt = b.sp[slot], sn = b.sn[slot];
-    V3 ro(so.x, so.y, so.z), rd(sd.x, sd.y, sd.z), pl(spt.x, spt.y, spt.z), nl(sn.x, sn.y, sn.z);
-    int medium = __float_as_int(so.w);
-    Lambda lam;
-    {
-        float4 l = b.lam[slot], lp = b.lpdf[slot];
-        lam = {{l.x, l.y, l.z, l.w}, {lp.x, lp.y, lp.z, lp.w}};
-    }
-    SS T(1.f);
-    for (int iter = 0;; ++iter) {
-        if (iter == 256) {
-            T = SS(0.f);
-            break;
-        }
-        DRay r{ro.x, ro.y, ro.z, rd.x, rd.y, rd.z};
-        DHit h;
-        if (!kInterfaces) {
-            if (dev_trace<true, kStats>(s.trace, r, kShadowTMax, &h, lds, tid, ts)) {
-                T = SS(0.f);
-            } else if (kMedia && medium >= 0) {
-                float l = len(rd);
-                T = T * medium_tr(s, medium, ro, rd / l, 1.f * l, lam);
-            }
-            break;
-        }
-        bool hit = dev_trace<false, kStats>(s.trace, r, kShadowTMax, &h, lds, tid, ts);
-        const prgpu::Primitive *pr = hit ? &s.prims[h.prim] : nullptr;
-        if (hit && !is_interface(s, *pr)) {
-            T = SS(0.f);
-            break;
-        }
-        if (kMedia && medium >= 0) {
-            float l = len(rd);
-            T = T * medium_tr(s, medium, ro, rd / l, (hit ? h.t : 1.f) * l, lam);
-        }
-        if (!T.nonzero() || !hit) break;
-        Surf si;
-        interaction(*pr, ro, rd, h.t, h.b1, h.b2, &si);
-        medium = dot(rd, si.n) > 0 ? pr->mediumOutside : pr->mediumInside;
-        ro = offset_origin(si.p, si.n, pl - si.p);
-        V3 target = offset_origin(pl, nl, ro - pl);
-        rd = target - ro;
-    }
-    if (!T.nonzero()) return;
-    shadow_add(b, slot, T, spt.w, sn.w);
-}
-
+// Transmittance of the shadow records in scenes with media or interfaces (src/scene/scene.cpp:41-59)
+// and the deferred add(): one any-hit query, or with interfaces a walk through their crossings (a
+// closest-hit query each), with the media's transmittance along the way. Persistent: a finished
+// query's lane goes on to its record's next segment or to another record.
 template <bool kStats, bool kMedia, bool kInterfaces>
 __global__ __launch_bounds__(kTraceBlock) void k_shadow(const DevScene *__restrict__ sp, Bufs b, const int *count,
                                                         int *fetch, unsigned long long *counters) {
     const DevScene &s = *sp;
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
-    const int n = *count;
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
-    TraceStats ts;
+    TraceStats st;
     uint32_t rays = 0;
-    if constexpr (!kMedia && !kInterfaces) {
-        int idx = -1, slot = 0;
-        bool started = false;
-        DRay r{};
-        TravState t{};
-        FetchState fs = fetch_begin();
-        while (fetch_rays_parts(fetch, n, idx, fs)) {
-            if (idx >= 0 && !started) {
-                slot = b.sq[idx];
-                float4 so = b.so[slot], sd = b.sd[slot];
-                r = DRay{so.x, so.y, so.z, sd.x, sd.y, sd.z};
-                trace_begin(t, r, kShadowTMax);
-                started = true;
-            }
-            if (!trace_turn(idx >= 0, t.cur)) continue;
-            if (trace_step<true, kStats>(s.trace, r, t, lds, tid, &ts)) {
-                ++rays;
-                if (!t.found) {
-                    float4 spk = b.sp[slot], snk = b.sn[slot];
-                    shadow_add(b, slot, SS(1.f), spk.w, snk.w);
-                }
-                idx = -1;
-                started = false;
-            }
-        }
-    } else {
-        const int stride = int(gridDim.x * blockDim.x);
-        for (int i = tid; i < n; i += stride) {
+    int slot = 0, medium = -1, iter = 0;
+    SS T(1.f);
+    trace_queue<kStats>(
+        s.trace, *count, fetch, lds, tid, &st,
+        [&](int i, DRay &r, TravState &t) {
+            slot = b.sq[i];
+            const float4 so = b.so[slot], sd = b.sd[slot];
+            r = DRay{so.x, so.y, so.z, sd.x, sd.y, sd.z};
+            medium = __float_as_int(so.w);
+            iter = 0;
+            T = SS(1.f);
+            trace_begin(t, r, kShadowTMax, !kInterfaces);
             ++rays;
-            shadow_walk<kMedia, kInterfaces, kStats>(s, b, b.sq[i], lds, tid, &ts);
-        }
-    }
+        },
+        [&](int, DRay &r, TravState &t) {
+            const bool hit = t.found();
+            if (!kInterfaces && hit) return false;
+            const prgpu::Primitive *pr = hit ? &s.prims[t.prim] : nullptr;
+            if (kInterfaces && hit && !is_interface(s, *pr)) return false;
+            const V3 ro(r.ox, r.oy, r.oz), rd(r.dx, r.dy, r.dz);
+            if (kMedia && medium >= 0) {
+                const float4 l4 = b.lam[slot], lp = b.lpdf[slot];
+                const Lambda lam = {{l4.x, l4.y, l4.z, l4.w}, {lp.x, lp.y, lp.z, lp.w}};
+                const float l = len(rd);
+                T = T * medium_tr(s, medium, ro, rd / l, (hit ? t.tMax : 1.f) * l, lam);
+            }
+            if (!T.nonzero()) return false;
+            const float4 spt = b.sp[slot], sn = b.sn[slot];
+            if (!kInterfaces || !hit) {
+                shadow_add(b, slot, T, spt.w, sn.w);
+                return false;
+            }
+            if (++iter == 256) return false;
+            const V3 pl(spt.x, spt.y, spt.z), nl(sn.x, sn.y, sn.z);
+            Surf si;
+            interaction(*pr, ro, rd, t.tMax, t.b1, t.b2, &si);
+            medium = dot(rd, si.n) > 0 ? pr->mediumOutside : pr->mediumInside;
+            const V3 o = offset_origin(si.p, si.n, pl - si.p);
+            const V3 d = offset_origin(pl, nl, o - pl) - o;
+            r = DRay{o.x, o.y, o.z, d.x, d.y, d.z};
+            trace_begin(t, r, kShadowTMax, false);
+            return true;
+        });
     if (kStats && rays) {
         atomicAdd(&counters[3], (unsigned long long)rays);
-        atomicAdd(&counters[4], (unsigned long long)ts.nodes);
-        atomicAdd(&counters[5], (unsigned long long)ts.recs);
+        atomicAdd(&counters[4], (unsigned long long)(st.nodes + st.anyNodes));
+        atomicAdd(&counters[5], (unsigned long long)(st.recs + st.anyRecs));
     }
 }
 
@@ -2353,7 +2265,7 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
     // launch (k_trace_bounce): a bounce appends them to shadow queue shadow_count_index(curIdx) and
     // the next one, whose curIdx is the other, consumes them. After the last bounce a round over the
     // empty path queue traces the last shadow rays.
-    const bool fused = kFusedShadow && !media && !interfaces;
+    const bool fused = !media && !interfaces;
     const bool sorted = dev.tune.materialSort != 0 && pt.sortable != 0;
     if (sorted) b.qk = pt.qk.as<int>();
     // The ray sort reorders the next queue into its own buffer, which the next bounce then traces
@@ -2373,7 +2285,7 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
             if (fused) {
                 auto *k = stats ? k_trace_bounce<true> : k_trace_bounce<false>;
                 hipLaunchKernelGGL(k, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, cur, b.counts + curIdx, b.counts + sIn,
-                                   b.counts + kFetchIntersect, b.counts + kFetchShadow, ctr);
+                                   b.counts + kFetchIntersect, ctr);
             } else if (stats) {
                 hipLaunchKernelGGL(k_intersect<true>, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, cur, b.counts + curIdx,
                                    b.counts + kFetchIntersect, ctr);
@@ -2436,9 +2348,9 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
         if (!fused)
             timer.Run(prgpu::KernShadow, 0, &pt.countsHost[2], [&] {
                 auto *k = stats ? (media ? (interfaces ? k_shadow<true, true, true> : k_shadow<true, true, false>)
-                                         : (interfaces ? k_shadow<true, false, true> : k_shadow<true, false, false>))
+                                         : k_shadow<true, false, true>)
                                 : (media ? (interfaces ? k_shadow<false, true, true> : k_shadow<false, true, false>)
-                                         : (interfaces ? k_shadow<false, false, true> : k_shadow<false, false, false>));
+                                         : k_shadow<false, false, true>);
                 hipLaunchKernelGGL(k, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, b.counts + 2, b.counts + kFetchShadow,
                                    ctr);
             });

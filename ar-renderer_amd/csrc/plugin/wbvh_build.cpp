@@ -169,10 +169,10 @@ class Collapser {
     WideBVH &out;
     explicit Collapser(const BinaryBuilder &b, WideBVH &o) : bb(b), out(o) {}
 
-    uint32_t Emit(int bn, int depth) {
+    // Fills node `self` (already allocated) from binary node bn and its subtree's nodes: the node's
+    // records first, then its internal children as one run of nodes.
+    void Emit(int self, int bn, int depth) {
         out.depth = std::max(out.depth, depth);
-        int self = int(out.nodes.size());
-        out.nodes.emplace_back();
         std::vector<int> kids;
         const BNode &root = bb.nodes[size_t(bn)];
         if (root.count > 0) {
@@ -198,28 +198,33 @@ class Collapser {
                 kids.insert(kids.begin() + best + 1, bb.nodes[size_t(open)].right);
             }
         }
-        uint32_t refs[8] = {0};
+        const uint32_t firstRec = uint32_t(out.recs.size()), firstNode = uint32_t(out.nodes.size());
+        uint8_t meta[8];
+        std::fill(meta, meta + 8, uint8_t(0x80));
+        int inner[8], nInner = 0;
         for (size_t i = 0; i < kids.size(); ++i) {
             const BNode &k = bb.nodes[size_t(kids[i])];
             if (k.count > 0) {
-                uint32_t first = uint32_t(out.recs.size());
+                meta[i] = uint8_t(0x80 + (out.recs.size() - firstRec));  // at most 7 x 8 records before it
                 for (int j = 0; j < k.count; ++j) out.recs.push_back(Record(bb.prims[size_t(k.first + j)].id));
-                refs[i] = kLeafBit | (uint32_t(k.count - 1) << 27) | first;
+                out.recs.back().prim |= kLastBit;
             } else {
-                refs[i] = Emit(kids[i], depth + 1);
+                meta[i] = uint8_t(nInner);
+                inner[nInner++] = kids[i];
             }
         }
+        out.nodes.resize(out.nodes.size() + size_t(nInner));
         WNode &w = out.nodes[size_t(self)];
         std::memset(&w, 0, sizeof(w));
-        w.nChildren = uint8_t(kids.size());
-        for (size_t i = 0; i < kids.size(); ++i) w.child[i] = refs[i];
+        w.childBase = firstNode;
+        w.recBase = (kLeafBit | firstRec) - 0x80u;
+        std::memcpy(w.meta, meta, 8);
         Quantise(kids, &w);
-        return uint32_t(self);
+        for (int i = 0; i < nInner; ++i) Emit(int(firstNode) + i, inner[i], depth + 1);
     }
 
     const prgpu::Primitive *prims = nullptr;
 
-  private:
     TriRec Record(int id) const {
         const prgpu::Primitive &p = prims[size_t(id)];
         TriRec r{};
@@ -262,13 +267,17 @@ class Collapser {
                     hi8[i] = uint8_t(qhi);
                 }
                 if (ok || e >= 127) {
-                    int8_t ee = int8_t(e);
+                    uint8_t ee = uint8_t(e + 127);  // 7 .. 254
                     if (a == 0) w->ex = ee;
                     if (a == 1) w->ey = ee;
                     if (a == 2) w->ez = ee;
                     for (size_t i = 0; i < kids.size(); ++i) {
                         w->qlo[a][i] = lo8[i];
                         w->qhi[a][i] = hi8[i];
+                    }
+                    for (size_t i = kids.size(); i < 8; ++i) {
+                        w->qlo[a][i] = 255;
+                        w->qhi[a][i] = 0;
                     }
                     break;
                 }
@@ -310,13 +319,27 @@ void BuildWideBVH(const prgpu::Primitive *prims, int count, WideBVH *out) {
         out->lo[a] = scene.lo[a];
         out->hi[a] = scene.hi[a];
     }
-    if (count == 0) return;
-    int root = bb.Build();
     Collapser c(bb, *out);
     c.prims = prims;
-    out->nodes.reserve(size_t(bb.used.load()) / 4 + 1);
-    out->recs.reserve(size_t(count));
-    c.Emit(root, 1);
+    if (count > 0) {
+        int root = bb.Build();
+        out->nodes.reserve(size_t(bb.used.load()) / 4 + 1);
+        out->recs.reserve(size_t(count) + 1);
+        out->nodes.resize(1);
+        c.Emit(0, root, 1);
+    } else {  // an empty scene: a root without children
+        out->nodes.resize(1);
+        WNode &w = out->nodes[0];
+        std::memset(&w, 0, sizeof(w));
+        w.ex = w.ey = w.ez = 127;
+        w.recBase = kLeafBit - 0x80u;
+        std::memset(w.meta, 0x80, sizeof(w.meta));
+        std::memset(w.qlo, 255, sizeof(w.qlo));
+        out->depth = 1;
+    }
+    TriRec none{};  // a triangle without extent: no ray hits it
+    none.prim = kLastBit;
+    out->recs.push_back(none);
 }
 
 }  // namespace pgpu
