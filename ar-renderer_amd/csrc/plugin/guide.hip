@@ -186,7 +186,8 @@ __device__ __forceinline__ void forward32(const GuideLds32 &L, const float *pos,
 
 // ---- inference -------------------------------------------------------------------------------
 // The decoded mixture (guide.h) for the queued vertices: queue[i] is a path slot whose hit record
-// (position h0, geometric normal h1) and incoming direction d describe the vertex; the mixture
+// (position h0, geometric normal h1) and incoming direction d (members of records of kVertexStride
+// float4) describe the vertex; the mixture
 // goes to out[12 i ..]. Vertex positions are normalised to the box (lo, inv extent).
 __global__ __launch_bounds__(kInferBlock) void k_guide_infer(const short *wt, const float *bias, const int *queue,
                                                              const int *count, const float4 *h0, const float4 *h1,
@@ -203,7 +204,8 @@ __global__ __launch_bounds__(kInferBlock) void k_guide_infer(const short *wt, co
         float pos[3] = {0.f, 0.f, 0.f}, nrm[3] = {0.f, 0.f, 0.f}, wo[3] = {0.f, 0.f, 0.f};
         if (valid) {
             const int slot = queue[idx];
-            float4 p = h0[slot], nn = h1[slot], d = dir[slot];
+            const size_t at = size_t(slot) * kVertexStride;
+            float4 p = h0[at], nn = h1[at], d = dir[at];
             pos[0] = (p.x - box.lo[0]) * box.inv[0];
             pos[1] = (p.y - box.lo[1]) * box.inv[1];
             pos[2] = (p.z - box.lo[2]) * box.inv[2];

@@ -14,6 +14,9 @@ struct GuideBox {
     float lo[3], inv[3];
 };
 
+// Members (float4) of the path-state records that inference reads.
+constexpr int kVertexStride = 4;
+
 struct GuideState {
     DevBuf params, m, v;   // FP32 master parameters and Adam moments
     DevBuf wt, bias;       // BF16 weights (Wt[out][in] per layer) and FP32 biases

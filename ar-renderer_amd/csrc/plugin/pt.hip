@@ -9,8 +9,9 @@
 // splats the samples of every pass onto the image with the film's reconstruction filter,
 // adding the pass value and its square to the FP64 sum and sum-of-squares accumulators.
 //
-// Path state is structure-of-arrays in HBM (float4 / int4 per field) so that the lanes of a
-// wave read and write consecutive 16-byte words.
+// Path state lives in 64-byte records by slot, each holding the four 16-byte fields that the same
+// kernels read and write (Bufs): a queue's slots grow sparse as paths end, and a path then costs the
+// memory sectors it uses rather than one sector per field.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -223,11 +224,12 @@ struct PTScene {
     std::vector<LNode> hostNodes;
     // batch buffers
     size_t cap = 0;
-    DevBuf o, d, rng, lam, lpdf, beta, rpath, L, Lh, prevP, prevN, st, hit, q0, q1, qm, qk, qms, sortBins, pfilm, xyz;
+    DevBuf ray, path, vertex, prev, shadow, shadowN, rpath, L, Lh;  // records and fields of the path state (see Bufs)
+    DevBuf q0, q1, qm, qk, qms, sortBins, pfilm, xyz;
     DevBuf nk, qr, raySortBins;
-    DevBuf h0, h1, h2, h3, qe, qeLpdf, qes;
+    DevBuf emit, qes;
     DevBuf sceneBuf;  // the DevScene the kernels read through a pointer
-    DevBuf so, sd, sp, sn, sf, sL, sb, sq;  // shadow records and the shadow queue
+    DevBuf sq;  // the shadow queue
     int *countsHost = nullptr;
     DevBuf counts;
     // The captured bounce rounds (see TraceBatch) and the key of what they were captured with.
@@ -695,13 +697,48 @@ struct Params {
     GuideBox box;      // the box vertex positions are normalised to for the model
 };
 
+// One field of the path state: element `slot` is a 16-byte member of a record of kStride members.
+template <class T, int kStride> struct Field {
+    T *p;
+    __device__ __forceinline__ T &operator[](int slot) const { return p[size_t(slot) * kStride]; }
+};
+using pgpu::ld4;
+using pgpu::st4;
+template <int kStride> __device__ __forceinline__ SS ld4(const Field<float4, kStride> &f, int i) {
+    const float4 v = f[i];
+    return {v.x, v.y, v.z, v.w};
+}
+template <int kStride> __device__ __forceinline__ void st4(const Field<float4, kStride> &f, int i, const SS &s) {
+    f[i] = make_float4(s.v[0], s.v[1], s.v[2], s.v[3]);
+}
+
+// The path state. Fields used together share a 64-byte record (one memory sector). The material and
+// surface stages are bound by the latency and volume of their reads: with an array per field, on the
+// gems scene (a fifth of the slots still alive after ten bounces) the material stage read 19.3 GB in
+// 8.1 ms and the surface stage 11.0 GB in 4.3 ms per pass; with records 9.3 GB in 4.2 ms and 6.9 GB in
+// 2.9 ms. Dense queues gain less (terrain: material 10.2 -> 9.2 ms per 16-spp call), and the camera
+// kernel, which only writes, loses (1.26 -> 1.56 ms).
 struct Bufs {
-    float4 *o, *d;
-    ulonglong2 *rng;
-    float4 *lam, *lpdf, *beta, *rpath, *L, *Lh, *prevP, *prevN;
-    int4 *st;
-    float4 *hit;
-    float4 *h0, *h1, *h2, *h3;  // surface hit records for the material stage
+    // ray record: traversal, surface stage
+    Field<float4, 4> o, d, hit;  // origin (w: prevPdf), direction (w: etaScale), hit
+    Field<int4, 4> st;           // depth, flags, medium, interface crossings; without media the surface
+                                 // stage leaves the depth to the material stage, which counts its vertex
+    // path record: material stage
+    Field<ulonglong2, 4> rng;
+    Field<float4, 4> beta, lam, lpdf;
+    // vertex record: surface hit for the material stage (or h0: a scattering point)
+    Field<float4, 4> h0, h1, h2, h3;
+    // the previous non-specular vertex, for the MIS weight of emission met from it
+    Field<float4, 2> prevP, prevN;
+    // Radiance, dense in the finish kernel. Without media the spectral-MIS ratios rpath stay 1, so L and
+    // the hero-wavelength sum Lh are the same and only L is kept.
+    float4 *rpath, *L, *Lh;
+    int media;
+    // shadow records, one per path slot (a path makes at most one shadow ray per bounce): origin (w:
+    // medium), direction, contribution before the transmittance; with media or interfaces also the light
+    // point (w: rpath average) and its normal
+    Field<float4, 4> so, sd, sc, sp;
+    float4 *sn;
     int *q0, *q1;
     int *qm;     // material queues, QCount x qcap
     int *qk;     // with the material sort: each material-queue entry's sort key (its material, or for a
@@ -719,15 +756,14 @@ struct Bufs {
                   // then the ray counters of the traversal and of the shadow walk (kFeedInts each)
     float2 *pfilm;
     float4 *xyz;
-    // shadow records, one per path slot (a path makes at most one shadow ray per bounce)
-    float4 *so, *sd, *sp, *sn, *sf, *sL, *sb;
     // guiding: decoded mixture per diffuse-queue entry (12 float4), kGuideRecords training
     // records per path (record j: 6 float4 planes of qcap at 6 j qcap: {position, state},
     // {normal, p_bsdf}, wo, w, throughput, radiance snapshot), compacted training records (16
     // floats) and their counter
     int *qes;       // emission queue (path slots)
-    int4 *qe;       // per slot: slot, depth and flags on arrival at the emitter, primitive (-1: escaped)
-    float4 *qeLpdf; // and the wavelength pdfs on arrival
+    Field<int4, 2> qe;  // per slot: 1 when qeLpdf holds the wavelength pdfs on arrival (the vertex ended
+                        // the secondary wavelengths), depth and flags on arrival, primitive (-1: escaped)
+    Field<float4, 2> qeLpdf;
     int *sq;        // shadow queue (path slots; the shadow records are indexed by slot)
     int shadowIdx;  // index in counts of the shadow queue's length this bounce appends to
     const float4 *gout;
@@ -915,11 +951,11 @@ __global__ __launch_bounds__(kBlock) void k_camera(const DevScene *__restrict__ 
     b.lam[slot] = make_float4(lam.l[0], lam.l[1], lam.l[2], lam.l[3]);
     b.lpdf[slot] = make_float4(lam.pdf[0], lam.pdf[1], lam.pdf[2], lam.pdf[3]);
     b.beta[slot] = make_float4(1, 1, 1, 1);
-    b.rpath[slot] = make_float4(1, 1, 1, 1);
     b.L[slot] = make_float4(0, 0, 0, 0);
-    b.Lh[slot] = make_float4(0, 0, 0, 0);
-    b.prevP[slot] = make_float4(0, 0, 0, 0);
-    b.prevN[slot] = make_float4(0, 0, 0, 0);
+    if (b.media) {
+        b.rpath[slot] = make_float4(1, 1, 1, 1);
+        b.Lh[slot] = make_float4(0, 0, 0, 0);
+    }
     b.st[slot] = make_int4(0, 0, s.cameraMedium, 0);
     b.pfilm[slot] = make_float2(fx, fy);
     b.q0[slot] = slot;
@@ -1036,14 +1072,13 @@ __device__ __forceinline__ bool sample_ld(const DevScene &s, const Bufs &b, int 
     V3 target = offset_origin(ls.pl, ls.nl, o - ls.pl);
     V3 d = target - o;
     int medium = kMedia ? (surface ? (dot(d, n) > 0 ? mOut : mIn) : r.medium) : -1;
-    const int rec = slot;
-    b.so[rec] = make_float4(o.x, o.y, o.z, __int_as_float(medium));
-    b.sd[rec] = make_float4(d.x, d.y, d.z, __int_as_float(slot));
-    b.sp[rec] = make_float4(ls.pl.x, ls.pl.y, ls.pl.z, k);
-    b.sn[rec] = make_float4(ls.nl.x, ls.nl.y, ls.nl.z, r.rpath.avg());
-    st4(b.sf, rec, f);
-    st4(b.sL, rec, ls.L);
-    st4(b.sb, rec, r.beta);
+    b.so[slot] = make_float4(o.x, o.y, o.z, __int_as_float(medium));
+    b.sd[slot] = make_float4(d.x, d.y, d.z, 0.f);
+    st4(b.sc, slot, r.beta * (f * ls.L * k));
+    if (kMedia || s.hasInterfaces) {
+        b.sp[slot] = make_float4(ls.pl.x, ls.pl.y, ls.pl.z, r.rpath.avg());
+        b.sn[slot] = make_float4(ls.nl.x, ls.nl.y, ls.nl.z, 0.f);
+    }
     return true;
 }
 
@@ -1097,15 +1132,11 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
     r.prevPdf = o.w;
     r.rd = V3(d.x, d.y, d.z);
     r.etaScale = d.w;
-    float4 lp = b.lpdf[slot];
-    const float4 lpIn = lp;
-    r.lam.pdf[0] = lp.x, r.lam.pdf[1] = lp.y, r.lam.pdf[2] = lp.z, r.lam.pdf[3] = lp.w;
     int4 st = b.st[slot];
     r.depth = st.x;
     r.flags = st.y;
     r.medium = st.z;
     r.crossings = st.w;
-    const bool lam0 = r.lam.terminated();
     // Training: the radiance gathered before this vertex closes the record of the guided
     // vertex the path just left (its own next-event estimate included).
     if (p.train)
@@ -1113,7 +1144,7 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
             const size_t base = 6 * j * size_t(b.qcap);
             float4 t0 = b.trec[base + slot];
             if (t0.w == 1.f) {
-                b.trec[base + 5 * size_t(b.qcap) + slot] = b.Lh[slot];
+                b.trec[base + 5 * size_t(b.qcap) + slot] = b.media ? b.Lh[slot] : b.L[slot];
                 t0.w = 2.f;
                 b.trec[base + slot] = t0;
             }
@@ -1128,8 +1159,8 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
     if (kMedia && r.medium >= 0) {
         // Distance sampling (path.cpp:159-191): the throughput and the spectral-MIS ratios take
         // the sample's weights; a scattering event moves the path to the phase-function queue.
-        float4 l = b.lam[slot];
-        r.lam.l[0] = l.x, r.lam.l[1] = l.y, r.lam.l[2] = l.z, r.lam.l[3] = l.w;
+        const float4 l = b.lam[slot], lp = b.lpdf[slot];
+        r.lam = {{l.x, l.y, l.z, l.w}, {lp.x, lp.y, lp.z, lp.w}};
         r.beta = ld4(b.beta, slot);
         r.rpath = ld4(b.rpath, slot);
         r.rng = load_rng(b, slot);
@@ -1157,6 +1188,7 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
     }
 
     const int depthIn = r.depth, flagsIn = r.flags;
+    bool dispersive = false;
     if (!done) {
         if (!hit) {
             emits = s.envCount > 0;
@@ -1172,6 +1204,8 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
                     interaction(pr, r.ro, r.rd, tHit, hv.z, hv.w, &si);
                     r.medium = dot(r.rd, si.n) > 0 ? pr.mediumOutside : pr.mediumInside;
                     r.ro = offset_origin(si.p, si.n, r.rd);
+                    b.o[slot] = make_float4(r.ro.x, r.ro.y, r.ro.z, r.prevPdf);
+                    if (!kMedia) b.st[slot] = make_int4(r.depth, r.flags, r.medium, r.crossings);
                 }
             } else if (!has_bsdf(s, pr)) {
                 alive = false;
@@ -1179,8 +1213,8 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
                 const prgpu::Material &m = s.mats[pr.material];
                 // A dispersive dielectric or coat keeps only the hero wavelength
                 // (material.cpp:106-110, 120-124), also when the depth limit ends the path here.
-                if (m.type == prgpu::MatDielectric && !spec_is_constant(s.spec, m.eta)) r.lam.terminate_secondary();
-                if (is_coated(m) && !spec_is_constant(s.spec, m.coatEta)) r.lam.terminate_secondary();
+                dispersive = (m.type == prgpu::MatDielectric && !spec_is_constant(s.spec, m.eta)) ||
+                             (is_coated(m) && !spec_is_constant(s.spec, m.coatEta));
                 if (r.depth++ >= p.maxDepth) {
                     alive = false;
                 } else {
@@ -1201,20 +1235,24 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
             }
         }
     }
+    bool ended = false;
+    float4 lpIn = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (dispersive) {
+        lpIn = b.lpdf[slot];
+        Lambda lam = {{0.f, 0.f, 0.f, 0.f}, {lpIn.x, lpIn.y, lpIn.z, lpIn.w}};
+        ended = !lam.terminated();
+        if (ended) {
+            lam.terminate_secondary();
+            b.lpdf[slot] = make_float4(lam.pdf[0], lam.pdf[1], lam.pdf[2], lam.pdf[3]);
+        }
+    }
     if (emits) {
         // The emission is evaluated with the wavelength pdfs and depth the path arrived with.
-        b.qe[slot] = make_int4(slot, depthIn, flagsIn, prim);
-        b.qeLpdf[slot] = lpIn;
+        b.qe[slot] = make_int4(ended ? 1 : 0, depthIn, flagsIn, prim);
+        if (ended) b.qeLpdf[slot] = lpIn;
         *q2 = QEmit;
     }
-
-    if (r.lam.terminated() != lam0)
-        b.lpdf[slot] = make_float4(r.lam.pdf[0], r.lam.pdf[1], r.lam.pdf[2], r.lam.pdf[3]);
-    b.st[slot] = make_int4(r.depth, r.flags, r.medium, r.crossings);
-    if (kMedia || kInterfaces) {
-        b.o[slot] = make_float4(r.ro.x, r.ro.y, r.ro.z, r.prevPdf);
-        b.d[slot] = make_float4(r.rd.x, r.rd.y, r.rd.z, r.etaScale);
-    }
+    if (kMedia) b.st[slot] = make_int4(r.depth, r.flags, r.medium, r.crossings);
     *q1 = toMaterial ? mq : (alive ? int(QNext) : -1);
     if (!toMaterial && alive && b.nk) *key = ray_key(p, r.ro, r.rd);
 }
@@ -1248,7 +1286,7 @@ __device__ __forceinline__ void emit_vertex(const DevScene &s, const Bufs &b, in
     const int4 e = b.qe[slot];
     const int prim = e.w;
     PathRegs r;
-    float4 o = b.o[slot], d = b.d[slot], l = b.lam[slot], lp = b.qeLpdf[slot];
+    float4 o = b.o[slot], d = b.d[slot], l = b.lam[slot], lp = e.x ? b.qeLpdf[slot] : b.lpdf[slot];
     r.ro = V3(o.x, o.y, o.z);
     r.prevPdf = o.w;
     r.rd = V3(d.x, d.y, d.z);
@@ -1256,9 +1294,13 @@ __device__ __forceinline__ void emit_vertex(const DevScene &s, const Bufs &b, in
     r.depth = e.y;
     r.flags = e.z;
     r.beta = ld4(b.beta, slot);
-    r.rpath = ld4(b.rpath, slot);
     r.L = ld4(b.L, slot);
-    r.Lh = ld4(b.Lh, slot);
+    r.rpath = SS(1.f);
+    r.Lh = SS(0.f);
+    if (b.media) {
+        r.rpath = ld4(b.rpath, slot);
+        r.Lh = ld4(b.Lh, slot);
+    }
     float4 pp = b.prevP[slot], pn = b.prevN[slot];
     r.prevP = V3(pp.x, pp.y, pp.z);
     r.prevN = V3(pn.x, pn.y, pn.z);
@@ -1279,7 +1321,7 @@ __device__ __forceinline__ void emit_vertex(const DevScene &s, const Bufs &b, in
         add_emitted(s, r, pr.light, area_L(s, s.lights[pr.light], si.n, -r.rd, r.lam), r.rd);
     }
     st4(b.L, slot, r.L);
-    st4(b.Lh, slot, r.Lh);
+    if (b.media) st4(b.Lh, slot, r.Lh);
 }
 
 __global__ __launch_bounds__(kBlock) void k_emit(const DevScene *__restrict__ sp, Bufs b) {
@@ -1305,9 +1347,9 @@ __device__ __forceinline__ void material_vertex(const DevScene &s, const Params 
     float4 l = b.lam[slot], lp = b.lpdf[slot];
     r.lam = {{l.x, l.y, l.z, l.w}, {lp.x, lp.y, lp.z, lp.w}};
     r.beta = ld4(b.beta, slot);
-    r.rpath = ld4(b.rpath, slot);
+    r.rpath = kMedia ? ld4(b.rpath, slot) : SS(1.f);
     int4 st = b.st[slot];
-    r.depth = st.x;
+    r.depth = kMedia ? st.x : st.x + 1;
     r.flags = st.y;
     r.medium = st.z;
     float4 h0 = b.h0[slot], h1 = b.h1[slot], h2 = b.h2[slot], h3 = b.h3[slot];
@@ -1407,8 +1449,10 @@ __device__ __forceinline__ void material_vertex(const DevScene &s, const Params 
         b.o[slot] = make_float4(r.ro.x, r.ro.y, r.ro.z, r.prevPdf);
         b.d[slot] = make_float4(r.rd.x, r.rd.y, r.rd.z, r.etaScale);
         st4(b.beta, slot, r.beta);
-        b.prevP[slot] = make_float4(si.p.x, si.p.y, si.p.z, 0.f);
-        b.prevN[slot] = make_float4(si.n.x, si.n.y, si.n.z, 0.f);
+        if (!(r.flags & kSpecularFlag)) {  // emission met after a specular bounce takes no MIS weight
+            b.prevP[slot] = make_float4(si.p.x, si.p.y, si.p.z, 0.f);
+            b.prevN[slot] = make_float4(si.n.x, si.n.y, si.n.z, 0.f);
+        }
         b.st[slot] = make_int4(r.depth, r.flags, r.medium, st.w);
         *q1 = QNext;
         if (b.nk) *key = ray_key(p, r.ro, r.rd);
@@ -1689,13 +1733,17 @@ __global__ __launch_bounds__(kBlock) void k_ray_sort_scatter(Bufs b, const int *
 // query's range is (0, 1 - 1e-4) in units of d (src/scene/interaction.h:43-47, scene.cpp:41-59).
 constexpr float kShadowTMax = 1 - 1e-4f;
 
-// The deferred add() of a visible shadow record: beta * (f * Tr * L * k), and the rPath
-// average at sampling time for the spectral-MIS estimate.
-__device__ __forceinline__ void shadow_add(const Bufs &b, int slot, const SS &T, float k, float a) {
-    SS c = ld4(b.sb, slot) * (ld4(b.sf, slot) * T * ld4(b.sL, slot) * k);
-    SS Lh = ld4(b.Lh, slot) + c;
-    st4(b.Lh, slot, Lh);
-    if (a > 0 && is_finite(a)) st4(b.L, slot, ld4(b.L, slot) + c / a);
+// The deferred add() of a visible shadow record: its contribution times the transmittance, and with
+// media the rPath average a at sampling time for the spectral-MIS estimate.
+__device__ __forceinline__ void shadow_add(const Bufs &b, int slot, const SS &T, float a) {
+    const SS c = ld4(b.sc, slot) * T;
+    if (b.media) {
+        st4(b.Lh, slot, ld4(b.Lh, slot) + c);
+        if (!(a > 0 && is_finite(a))) return;
+        st4(b.L, slot, ld4(b.L, slot) + c / a);
+    } else {
+        st4(b.L, slot, ld4(b.L, slot) + c);
+    }
 }
 
 // Closest hits of the current queue and, in the same persistent launch, the shadow rays of the
@@ -1732,10 +1780,7 @@ __global__ __launch_bounds__(kTraceBlock) PG_WAVES(8) void k_trace_bounce(const 
         [&](int, DRay &, TravState &t) {
             if (t.any) {
                 ++raysS;
-                if (!t.found()) {
-                    const float4 spk = b.sp[slot], snk = b.sn[slot];
-                    shadow_add(b, slot, SS(1.f), spk.w, snk.w);
-                }
+                if (!t.found()) shadow_add(b, slot, SS(1.f), 1.f);
             } else {
                 ++raysC;
                 b.hit[slot] = closest_hit(t);
@@ -1791,12 +1836,13 @@ __global__ __launch_bounds__(kTraceBlock) void k_shadow(const DevScene *__restri
                 T = T * medium_tr(s, medium, ro, rd / l, (hit ? t.tMax : 1.f) * l, lam);
             }
             if (!T.nonzero()) return false;
-            const float4 spt = b.sp[slot], sn = b.sn[slot];
+            const float4 spt = b.sp[slot];
             if (!kInterfaces || !hit) {
-                shadow_add(b, slot, T, spt.w, sn.w);
+                shadow_add(b, slot, T, spt.w);
                 return false;
             }
             if (++iter == 256) return false;
+            const float4 sn = b.sn[slot];
             const V3 pl(spt.x, spt.y, spt.z), nl(sn.x, sn.y, sn.z);
             Surf si;
             interaction(*pr, ro, rd, t.tMax, t.b1, t.b2, &si);
@@ -1822,7 +1868,7 @@ __global__ __launch_bounds__(kBlock) void k_finish(const DevScene *__restrict__ 
     if (slot >= n) return;
     float4 lp = b.lpdf[slot], l = b.lam[slot];
     Lambda lam = {{l.x, l.y, l.z, l.w}, {lp.x, lp.y, lp.z, lp.w}};
-    SS L = lam.terminated() ? ld4(b.Lh, slot) : ld4(b.L, slot);
+    SS L = b.media && lam.terminated() ? ld4(b.Lh, slot) : ld4(b.L, slot);
     L = L * 1.f;  // camera ray weight
     if (p.train)
         for (int r = 0; r < kGuideRecords; ++r) {
@@ -1832,7 +1878,7 @@ __global__ __launch_bounds__(kBlock) void k_finish(const DevScene *__restrict__ 
             const size_t c = size_t(b.qcap);
             const float4 *t = b.trec + 6 * r * c;
             if (t[slot].w != 2.f) continue;
-            const SS Lh = ld4(b.Lh, slot), snap = ld4(t, 5 * c + slot), beta0 = ld4(t, 4 * c + slot);
+            const SS Lh = ld4(b.media ? b.Lh : b.L, slot), snap = ld4(t, 5 * c + slot), beta0 = ld4(t, 4 * c + slot);
             float w = 0.f;
             int k = 0;
             for (int j = 0; j < 4; ++j)
@@ -2068,10 +2114,13 @@ __global__ __launch_bounds__(kBlock) void k_gather_tiled(const DevScene *__restr
 
 void EnsureBatch(PTScene &pt, size_t n) {
     if (pt.cap >= n) return;
-    auto f4 = [&](DevBuf &b) { b.ensure(n * sizeof(float4)); };
-    f4(pt.o); f4(pt.d); f4(pt.lam); f4(pt.lpdf); f4(pt.beta); f4(pt.rpath); f4(pt.L); f4(pt.Lh);
-    f4(pt.prevP); f4(pt.prevN); f4(pt.hit); f4(pt.xyz);
-    f4(pt.h0); f4(pt.h1); f4(pt.h2); f4(pt.h3); f4(pt.qe); f4(pt.qeLpdf);
+    auto f4 = [&](DevBuf &b, size_t members) { b.ensure(n * members * sizeof(float4)); };
+    f4(pt.ray, 4); f4(pt.path, 4); f4(pt.vertex, 4); f4(pt.prev, 2); f4(pt.shadow, 4); f4(pt.emit, 2);
+    f4(pt.L, 1); f4(pt.xyz, 1);
+    if (pt.hasMedia) {
+        f4(pt.rpath, 1); f4(pt.Lh, 1);
+    }
+    if (pt.hasMedia || pt.hasInterfaces) f4(pt.shadowN, 1);
     pt.qes.ensure(n * sizeof(int));
     pt.sq.ensure(n * sizeof(int));
     pt.qm.ensure(n * QCount * sizeof(int));
@@ -2087,9 +2136,6 @@ void EnsureBatch(PTScene &pt, size_t n) {
         pt.raySortBins.ensure(2 * kRaySortBins * sizeof(int));
         PG_CHECK(hipMemset(pt.raySortBins.p, 0, pt.raySortBins.bytes));
     }
-    f4(pt.so); f4(pt.sd); f4(pt.sp); f4(pt.sn); f4(pt.sf); f4(pt.sL); f4(pt.sb);
-    pt.rng.ensure(n * sizeof(ulonglong2));
-    pt.st.ensure(n * sizeof(int4));
     pt.q0.ensure(n * sizeof(int));
     pt.q1.ensure(n * sizeof(int));
     pt.pfilm.ensure(n * sizeof(float2));
@@ -2098,12 +2144,17 @@ void EnsureBatch(PTScene &pt, size_t n) {
 
 Bufs MakeBufs(PTScene &pt) {
     Bufs b{};  // zeroed, padding included: the bounce-graph key hashes its bytes
-    b.o = pt.o.as<float4>(); b.d = pt.d.as<float4>(); b.rng = pt.rng.as<ulonglong2>();
-    b.lam = pt.lam.as<float4>(); b.lpdf = pt.lpdf.as<float4>(); b.beta = pt.beta.as<float4>();
+    float4 *ray = pt.ray.as<float4>(), *path = pt.path.as<float4>(), *vertex = pt.vertex.as<float4>();
+    b.o.p = ray; b.d.p = ray + 1; b.hit.p = ray + 2; b.st.p = reinterpret_cast<int4 *>(ray + 3);
+    b.rng.p = reinterpret_cast<ulonglong2 *>(path); b.beta.p = path + 1; b.lam.p = path + 2; b.lpdf.p = path + 3;
+    b.h0.p = vertex; b.h1.p = vertex + 1; b.h2.p = vertex + 2; b.h3.p = vertex + 3;
+    b.prevP.p = pt.prev.as<float4>(); b.prevN.p = b.prevP.p + 1;
     b.rpath = pt.rpath.as<float4>(); b.L = pt.L.as<float4>(); b.Lh = pt.Lh.as<float4>();
-    b.prevP = pt.prevP.as<float4>(); b.prevN = pt.prevN.as<float4>(); b.st = pt.st.as<int4>();
-    b.hit = pt.hit.as<float4>(); b.q0 = pt.q0.as<int>(); b.q1 = pt.q1.as<int>(); b.counts = pt.counts.as<int>();
-    b.h0 = pt.h0.as<float4>(); b.h1 = pt.h1.as<float4>(); b.h2 = pt.h2.as<float4>(); b.h3 = pt.h3.as<float4>();
+    b.media = pt.hasMedia;
+    b.so.p = pt.shadow.as<float4>(); b.sd.p = b.so.p + 1; b.sc.p = b.so.p + 2; b.sp.p = b.so.p + 3;
+    b.sn = pt.shadowN.as<float4>();
+    b.qe.p = pt.emit.as<int4>(); b.qeLpdf.p = pt.emit.as<float4>() + 1;
+    b.q0 = pt.q0.as<int>(); b.q1 = pt.q1.as<int>(); b.counts = pt.counts.as<int>();
     b.qm = pt.qm.as<int>();
     b.qk = nullptr;  // set by a batch that sorts the material queues
     b.qms = pt.qms.as<int>();
@@ -2116,12 +2167,8 @@ Bufs MakeBufs(PTScene &pt) {
     b.qes = pt.qes.as<int>();
     b.sq = pt.sq.as<int>();
     b.shadowIdx = 2;
-    b.qe = pt.qe.as<int4>();
-    b.qeLpdf = pt.qeLpdf.as<float4>();
     b.qcap = int(pt.cap);
     b.pfilm = pt.pfilm.as<float2>(); b.xyz = pt.xyz.as<float4>();
-    b.so = pt.so.as<float4>(); b.sd = pt.sd.as<float4>(); b.sp = pt.sp.as<float4>(); b.sn = pt.sn.as<float4>();
-    b.sf = pt.sf.as<float4>(); b.sL = pt.sL.as<float4>(); b.sb = pt.sb.as<float4>();
     b.gout = nullptr;
     b.trec = nullptr;
     b.train = nullptr;
@@ -2313,8 +2360,8 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
         if (sorted) mb.qm = b.qms;
         if (guided)
             timer.Run(prgpu::KernGuide, 0, nullptr, [&] {
-                dev.guide->Infer(mb.qm + size_t(QDiffuse) * b.qcap, b.counts + mat_count_index(QDiffuse), active, b.h0,
-                                 b.h1, b.d, p.box, dev.cus, st);
+                dev.guide->Infer(mb.qm + size_t(QDiffuse) * b.qcap, b.counts + mat_count_index(QDiffuse), active, b.h0.p,
+                                 b.h1.p, b.d.p, p.box, dev.cus, st);
             });
         timer.Run(prgpu::KernMaterial, active, nullptr, [&] {
             if (guided) {
