@@ -220,8 +220,6 @@ struct PTScene {
     int hasInterfaces = 0, hasMedia = 0, hasLayered = 0;  // hasLayered: coated or sheen materials
     int sortable = 0;  // more than one material or medium: the material sort can group anything
     float cieYInt = 1;
-    // host copies for inspection
-    std::vector<LNode> hostNodes;
     // batch buffers
     size_t cap = 0;
     DevBuf ray, path, vertex, prev, shadow, shadowN, rpath, L, Lh;  // records and fields of the path state (see Bufs)
@@ -538,19 +536,19 @@ void EnsurePTScene(Device &dev, const prgpu::SceneDescEx &sd, const float *sheen
     for (size_t i = 0; i < nodes.size(); ++i) {
         LNode &n = nodes[i];
         const HostLB &x = tb.lbs[i];
-        n.lo[0] = x.bounds.lo.x; n.lo[1] = x.bounds.lo.y; n.lo[2] = x.bounds.lo.z;
-        n.hi[0] = x.bounds.hi.x; n.hi[1] = x.bounds.hi.y; n.hi[2] = x.bounds.hi.z;
+        n.SetBounds(x.bounds.lo, x.bounds.hi);
         n.w[0] = x.w.x; n.w[1] = x.w.y; n.w[2] = x.w.z;
         n.phi = x.phi;
         n.cosTheta_o = x.cosTheta_o;
+        n.sinTheta_o = safe_sqrt(1 - sq(x.cosTheta_o));
         n.cosTheta_e = x.cosTheta_e;
         n.child1 = tb.child1[i];
         n.light = tb.light[i];
-        n.parent = tb.parent[i];
-        n.twoSided = x.twoSided ? 1u : 0u;
+        const int par = tb.parent[i];
+        n.parent = 2 * par + (x.twoSided ? 1 : 0);
+        n.sibling = par < 0 ? -1 : (int(i) == par + 1 ? tb.child1[size_t(par)] : par + 1);
         if (n.light >= 0) leafOf[size_t(n.light)] = int(i);
     }
-    pt->hostNodes = nodes;
     pt->lnodeCount = int(nodes.size());
     if (nodes.empty()) nodes.push_back(LNode{});  // no bounded lights: a placeholder the kernels never read
     pt->lnodes.upload(nodes.data(), nodes.size(), s);

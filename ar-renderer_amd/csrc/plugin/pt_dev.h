@@ -94,7 +94,7 @@ PG_HD V3 cosine_hemisphere(V2 u) {
 }
 PG_HD V3 uniform_sphere(V2 u) {
     float z = 1 - 2 * u.x;
-    float r = safe_sqrt(1 - z * z);
+    float r = sqrt_1m(z * z);
     float phi = 2 * kPi * u.y;
     return {r * cosf(phi), r * sinf(phi), z};
 }
@@ -293,7 +293,7 @@ PG_HD float fr_dielectric(float ci, float eta) {
     float s2i = 1 - sq(ci);
     float s2t = s2i / sq(eta);
     if (s2t >= 1) return 1.f;
-    float ct = safe_sqrt(1 - s2t);
+    float ct = sqrt_1m(s2t);
     float rpa = (eta * ci - ct) / (eta * ci + ct);
     float rpe = (ci - eta * ct) / (ci + eta * ct);
     return (sq(rpa) + sq(rpe)) / 2;
@@ -1408,29 +1408,29 @@ PG_HD int light_sample(const DevScene &s, V3 p, V3 n, float u, float *pmf) {
     }
     if (s.lnodeCount == 0) return -1;
     u = minf((u - pInf) / (1 - pInf), kOneMinusEps);
-    int ni = 0;
+    // Descends by the two children's importances. A child's tail (its children, light) comes with the
+    // record its importance is read from, so a level is one round of loads.
+    int ni = 0, light = s.lnodes[0].light, child1 = s.lnodes[0].child1;
     float prob = 1 - pInf;
     for (int guard = 0; guard < 64; ++guard) {
-        const LNode &node = s.lnodes[ni];
-        if (node.light >= 0) {
-            if (ni > 0 || lb_importance(node, p, n) > 0) {
+        if (light >= 0) {
+            if (ni > 0 || lb_importance(s.lnodes[0], p, n) > 0) {
                 *pmf = prob;
-                return node.light;
+                return light;
             }
             return -1;
         }
-        float ci0 = lb_importance(s.lnodes[ni + 1], p, n), ci1 = lb_importance(s.lnodes[node.child1], p, n);
+        const LNode a = s.lnodes[ni + 1], b = s.lnodes[child1];
+        float ci0 = lb_importance(a, p, n), ci1 = lb_importance(b, p, n);
         if (ci0 == 0 && ci1 == 0) return -1;
         float p0 = ci0 / (ci0 + ci1);
-        if (u < p0) {
-            prob *= p0;
-            u = minf(u / p0, kOneMinusEps);
-            ni = ni + 1;
-        } else {
-            prob *= 1 - p0;
-            u = minf((u - p0) / (1 - p0), kOneMinusEps);
-            ni = node.child1;
-        }
+        const bool first = u < p0;
+        const float q = first ? p0 : 1 - p0;
+        prob *= q;
+        u = minf((first ? u : u - p0) / q, kOneMinusEps);
+        ni = first ? ni + 1 : child1;
+        light = first ? a.light : b.light;
+        child1 = first ? a.child1 : b.child1;
     }
     return -1;
 }
@@ -1446,12 +1446,12 @@ PG_HD float light_pmf(const DevScene &s, V3 p, V3 n, int li) {
     }
     if (leaf == 0) return lb_importance(s.lnodes[0], p, n) > 0 ? 1 - p_infinite(s) : 0.f;
     float pm = 1 - p_infinite(s);
-    for (int child = leaf, par = s.lnodes[leaf].parent, guard = 0; par >= 0 && guard < 64;
-         child = par, par = s.lnodes[par].parent, ++guard) {
-        const LNode &node = s.lnodes[par];
-        float ci0 = lb_importance(s.lnodes[par + 1], p, n), ci1 = lb_importance(s.lnodes[node.child1], p, n);
-        if (ci0 == 0 && ci1 == 0) return 0;
-        pm *= (child == node.child1 ? ci1 : ci0) / (ci0 + ci1);
+    for (int child = leaf, guard = 0; child > 0 && guard < 64; ++guard) {
+        const LNode a = s.lnodes[child];
+        const float ca = lb_importance(a, p, n), cb = lb_importance(s.lnodes[a.sibling], p, n);
+        if (ca == 0 && cb == 0) return 0;
+        pm *= ca / (ca + cb);
+        child = a.parent >> 1;
     }
     return pm;
 }
