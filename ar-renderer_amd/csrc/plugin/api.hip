@@ -254,25 +254,21 @@ void LaunchTraceRays(Device &d, const TraceCtx &c, uint32_t *words, bool clearFl
 // The reference keys its upload cache on the host pointer and counts only; a strided content
 // sample additionally catches buffers that are reused with new contents.
 uint64_t GeometryKey(const prgpu::Primitive *prims, int count) {
-    uint64_t h = 1469598103934665603ull;
-    auto mix = [&](const void *p, size_t n) {
-        const unsigned char *b = static_cast<const unsigned char *>(p);
-        for (size_t i = 0; i < n; ++i) h = (h ^ b[i]) * 1099511628211ull;
-    };
-    mix(&count, sizeof(count));
-    uintptr_t ptr = uintptr_t(prims);
-    mix(&ptr, sizeof(ptr));
+    ContentKey k;
+    const uintptr_t head[2] = {uintptr_t(count), uintptr_t(prims)};
+    k.Mix(head, sizeof(head));
     if (count > 0) {
-        int step = std::max(1, count / 4096);
-        for (int i = 0; i < count; i += step) mix(&prims[i], sizeof(prgpu::Primitive));
-        mix(&prims[count - 1], sizeof(prgpu::Primitive));
+        const int step = std::max(1, count / 4096);
+        for (int64_t i = 0; i < count; i += step) k.Mix(&prims[i], sizeof(prgpu::Primitive));
+        k.Mix(&prims[count - 1], sizeof(prgpu::Primitive));
     }
-    return h;
+    return k.Value();
 }
 
-void EnsureGeometry(Device &d, const prgpu::Primitive *prims, int count) {
-    uint64_t key = GeometryKey(prims, count);
-    if (key == d.geomKey && d.nodes.p) return;
+uint64_t EnsureGeometry(Device &d, const prgpu::Primitive *prims, int count) {
+    const uint64_t key = GeometryKey(prims, count);
+    if (key == d.geomKey && d.nodes.p) return key;
+    d.geomKey = 0;
     WideBVH bvh;
     BuildWideBVH(prims, count, &bvh);
     d.nodes.upload(bvh.nodes.data(), bvh.nodes.size(), d.stream);
@@ -291,6 +287,7 @@ void EnsureGeometry(Device &d, const prgpu::Primitive *prims, int count) {
     if (d.spillCap > 0) d.spill.ensure(size_t(d.spillCap) * size_t(d.spillStride) * sizeof(uint32_t));
     PG_CHECK(hipStreamSynchronize(d.stream));
     d.geomKey = key;
+    return key;
 }
 
 TraceCtx MakeTraceCtx(Device &d) {
@@ -475,8 +472,7 @@ PRGPU_API int prgpu_render_ex(int deviceIndex, const prgpu::SceneDescEx *sd, con
             throw std::runtime_error("API version mismatch");
         if (!rp || (!sum && sumsq)) throw std::runtime_error("invalid arguments");
         Device &d = Get(deviceIndex);
-        EnsureGeometry(d, sd->prims, sd->primCount);
-        RenderExImpl(d, *sd, *rp, sum, sumsq);
+        RenderExImpl(d, EnsureGeometry(d, sd->prims, sd->primCount), *sd, *rp, sum, sumsq);
         return 0;
     } catch (const std::exception &e) {
         SetErr(err, errLen, e.what());
@@ -493,8 +489,7 @@ PRGPU_API int prgpu_sample_radiance(int deviceIndex, const prgpu::SceneDescEx *s
             throw std::runtime_error("API version mismatch");
         if (!rp || !out) throw std::runtime_error("invalid arguments");
         Device &d = Get(deviceIndex);
-        EnsureGeometry(d, sd->prims, sd->primCount);
-        SampleRadianceImpl(d, *sd, *rp, out);
+        SampleRadianceImpl(d, EnsureGeometry(d, sd->prims, sd->primCount), *sd, *rp, out);
         return 0;
     } catch (const std::exception &e) {
         SetErr(err, errLen, e.what());
@@ -617,6 +612,9 @@ PRGPU_API int prgpu_release(int deviceIndex) {
     d.spill.release();
     d.rays.release();
     d.hits.release();
+    d.hostSum.release();
+    d.hostSq.release();
+    d.records.release();
     d.filmSum.release();
     d.filmSq.release();
     d.filmW = d.filmH = 0;
@@ -670,11 +668,10 @@ PRGPU_API int prgpu_guide_eval(int deviceIndex, const float *records, int n, flo
         Device &d = Get(deviceIndex);
         pgpu::GuideState &g = EnsureGuide(d);
         if (n == 0) return 0;
-        DevBuf in, out;
-        in.upload(records, size_t(n) * 9, d.stream);
-        out.ensure(size_t(n) * pgpu::kGOut * sizeof(float));
-        g.Eval(in.as<float>(), n, out.as<float>(), d.stream);
-        PG_CHECK(hipMemcpyAsync(out41, out.p, size_t(n) * pgpu::kGOut * sizeof(float), hipMemcpyDeviceToHost, d.stream));
+        g.in.upload(records, size_t(n) * 9, d.stream);
+        g.eval.ensure(size_t(n) * pgpu::kGOut * sizeof(float));
+        g.Eval(g.in.as<float>(), n, g.eval.as<float>(), d.stream);
+        PG_CHECK(hipMemcpyAsync(out41, g.eval.p, size_t(n) * pgpu::kGOut * sizeof(float), hipMemcpyDeviceToHost, d.stream));
         PG_CHECK(hipStreamSynchronize(d.stream));
         return 0;
     } catch (const std::exception &) {
@@ -691,13 +688,12 @@ PRGPU_API int prgpu_guide_train(int deviceIndex, const float *records, int n, in
         Device &d = Get(deviceIndex);
         pgpu::GuideState &g = EnsureGuide(d);
         g.blend = d.tune.guideBlend;
-        DevBuf in;
-        in.upload(records, size_t(n) * 16, d.stream);
+        g.in.upload(records, size_t(n) * 16, d.stream);
         if (steps == 0) {
-            g.Gradient(in.as<float>(), nullptr, 0, n, d.stream);
+            g.Gradient(g.in.as<float>(), nullptr, 0, n, d.stream);
             PG_CHECK(hipMemcpyAsync(grad, g.grad.p, size_t(pgpu::kGParams) * sizeof(float), hipMemcpyDeviceToHost, d.stream));
         } else {
-            for (int k = 0; k < steps; ++k) g.Step(in.as<float>(), nullptr, 0, n, lr, d.stream);
+            for (int k = 0; k < steps; ++k) g.Step(g.in.as<float>(), nullptr, 0, n, lr, d.stream);
         }
         if (stats) PG_CHECK(hipMemcpyAsync(stats, g.stats.p, 2 * sizeof(float), hipMemcpyDeviceToHost, d.stream));
         PG_CHECK(hipStreamSynchronize(d.stream));

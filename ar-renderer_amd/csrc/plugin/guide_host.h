@@ -22,6 +22,7 @@ struct GuideState {
     DevBuf wt, bias;       // BF16 weights (Wt[out][in] per layer) and FP32 biases
     DevBuf grad, stats, part;
     DevBuf out, rec;       // per batch: raw outputs per guided vertex, training record per path
+    DevBuf in, eval;       // staging of the probes' host arrays, kept with the model
     DevBuf train, trainCount;  // compacted training records; [0] written, [1] produced
     size_t cap = 0, trainCap = 0;
     int steps = 0;

@@ -220,6 +220,7 @@ struct PTScene {
     int hasInterfaces = 0, hasMedia = 0, hasLayered = 0;  // hasLayered: coated or sheen materials
     int sortable = 0;  // more than one material or medium: the material sort can group anything
     float cieYInt = 1;
+    float filterRadius = 0.5f, filterSigma = 0.5f, filterNorm = 1;
     // batch buffers
     size_t cap = 0;
     DevBuf ray, path, vertex, prev, shadow, shadowN, rpath, L, Lh;  // records and fields of the path state (see Bufs)
@@ -253,12 +254,10 @@ void ReleasePT(Device &d) {
 
 namespace {
 
-uint64_t PTKey(const prgpu::SceneDescEx &sd, const float *sheenTable) {
-    uint64_t h = 1469598103934665603ull;
-    auto mix = [&](const void *p, size_t n) {
-        const unsigned char *b = static_cast<const unsigned char *>(p);
-        for (size_t i = 0; i < n; ++i) h = (h ^ b[i]) * 1099511628211ull;
-    };
+uint64_t PTKey(uint64_t geomKey, const prgpu::SceneDescEx &sd, const float *sheenTable) {
+    ContentKey k;
+    auto mix = [&](const void *p, size_t n) { k.Mix(p, n); };
+    mix(&geomKey, sizeof(geomKey));
     mix(&sd.primCount, sizeof(int));
     if (sd.materialCount) mix(sd.materials, sizeof(prgpu::Material) * size_t(sd.materialCount));
     if (sd.spectrumCount) mix(sd.spectra, sizeof(prgpu::SpectrumEx) * size_t(sd.spectrumCount));
@@ -273,7 +272,7 @@ uint64_t PTKey(const prgpu::SceneDescEx &sd, const float *sheenTable) {
     mix(&sd.cameraMedium, sizeof(int));
     mix(&sd.camera, sizeof(sd.camera));
     if (sheenTable) mix(sheenTable, sizeof(float) * prgpu::kSheenAlpha * prgpu::kSheenMu);
-    return h ^ GeometryKey(sd.prims, sd.primCount);
+    return k.Value();
 }
 
 void Validate(const prgpu::SceneDescEx &sd) {
@@ -414,11 +413,13 @@ const std::vector<float> &HostSheenTable() {
     return t;
 }
 
-void EnsurePTScene(Device &dev, const prgpu::SceneDescEx &sd, const float *sheenTable) {
+float FilterEval1D(int type, float radius, float sigma, float x);
+
+void EnsurePTScene(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, const float *sheenTable) {
     // The traversal reads the device-resident BVH: it must be this scene's.
-    if (!dev.nodes.p || dev.geomKey != GeometryKey(sd.prims, sd.primCount))
+    if (!dev.nodes.p || dev.geomKey != geomKey)
         throw std::runtime_error("internal error: the scene's geometry is not on the device");
-    uint64_t key = PTKey(sd, sheenTable);
+    const uint64_t key = PTKey(geomKey, sd, sheenTable);
     if (dev.pt && dev.ptKey == key) return;
     Validate(sd);
     dev.guide.reset();  // a model learned for another scene
@@ -595,6 +596,20 @@ void EnsurePTScene(Device &dev, const prgpu::SceneDescEx &sd, const float *sheen
     pt->hasMedia = (sd.cameraMedium >= 0) ? 1 : 0;
     for (int i = 0; i < sd.primCount && !pt->hasMedia; ++i)
         if (sd.prims[i].mediumInside >= 0 || sd.prims[i].mediumOutside >= 0) pt->hasMedia = 1;
+    // Film filter (src/core/film.cpp:9-22, 42): its norm integrates the profile over 4096 points.
+    {
+        const int ft = sd.camera.filterType;
+        float r = sd.camera.filterRadius, sigma = 0.5f;
+        if (ft == prgpu::FilterBox) r = std::max(0.5f, std::min(r, 0.5f));
+        if (ft == prgpu::FilterGaussian) sigma = r / 3.f;
+        const int n = 4096;
+        double s1 = 0;
+        for (int i = 0; i < n; ++i) s1 += FilterEval1D(ft, r, sigma, -r + (i + 0.5f) * (2 * r / n));
+        s1 *= 2 * r / n;
+        pt->filterRadius = r;
+        pt->filterSigma = sigma;
+        pt->filterNorm = float(1.0 / (s1 * s1));
+    }
     PG_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pt->countsHost), kCountsBytes, hipHostMallocDefault));
     pt->counts.ensure(kCountsBytes);
     PG_CHECK(hipMemsetAsync(pt->counts.p, 0, kCountsBytes, s));
@@ -654,20 +669,11 @@ DevScene MakeDevScene(Device &dev, const prgpu::SceneDescEx &sd, const prgpu::Re
     s.width = sd.camera.width;
     s.height = sd.camera.height;
     // Film filter and margin (src/core/film.cpp:9-22, 42).
-    int ft = sd.camera.filterType;
-    float r = sd.camera.filterRadius;
-    float sigma = 0.5f;
-    if (ft == prgpu::FilterBox) r = std::max(0.5f, std::min(r, 0.5f));
-    if (ft == prgpu::FilterGaussian) sigma = r / 3.f;
-    const int n = 4096;
-    double s1 = 0;
-    for (int i = 0; i < n; ++i) s1 += FilterEval1D(ft, r, sigma, -r + (i + 0.5f) * (2 * r / n));
-    s1 *= 2 * r / n;
-    s.filterType = ft;
-    s.filterRadius = r;
-    s.filterSigma = sigma;
-    s.filterNorm = float(1.0 / (s1 * s1));
-    s.margin = int(std::ceil(r - 0.5f));
+    s.filterType = sd.camera.filterType;
+    s.filterRadius = pt.filterRadius;
+    s.filterSigma = pt.filterSigma;
+    s.filterNorm = pt.filterNorm;
+    s.margin = int(std::ceil(pt.filterRadius - 0.5f));
     s.xyzNorm = 1.f / (4 * pt.cieYInt);
     s.trace = MakeTraceCtx(dev);
     return s;
@@ -2464,7 +2470,6 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
             ++k;
             if (bound == 0) break;  // round k (queued, empty) is the last
         }
-        PG_CHECK(hipStreamSynchronize(st));
     } else {
         int curIdx = 0, bounce = 0;
         // A round runs while paths remain or, with fused shadow rays, while the last round left
@@ -2496,25 +2501,32 @@ int PassesPerBatch(const Device &dev, int npix, int spp) {
 
 }  // namespace
 
-void RenderExImpl(Device &dev, const prgpu::SceneDescEx &sd, const prgpu::RenderParamsEx &rp, double *sum,
-                  double *sumsq, const float *sheenTable) {
-    if (rp.spp <= 0) return;
-    EnsurePTScene(dev, sd, sheenTable);
+void RenderExImpl(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, const prgpu::RenderParamsEx &rp, double *sum,
+                  double *sumsq, bool fromZero, const float *sheenTable) {
+    const size_t filmN = size_t(std::max(0, sd.camera.width)) * size_t(std::max(0, sd.camera.height)) * 3;
+    if (rp.spp <= 0) {
+        if (sum && fromZero) std::fill(sum, sum + filmN, 0.0);
+        return;
+    }
+    EnsurePTScene(dev, geomKey, sd, sheenTable);
     DevScene s = MakeDevScene(dev, sd, rp);
     const DevScene *ds = UploadDevScene(dev, s);
     const int sw = s.width + 2 * s.margin, sh = s.height + 2 * s.margin, npix = sw * sh;
     const int per = PassesPerBatch(dev, npix, rp.spp);
     PTScene &pt = *dev.pt;
     EnsureBatch(pt, size_t(per) * size_t(npix));
-    const size_t filmN = size_t(s.width) * s.height * 3;
     // Host film: stage it in HBM for the call. Resident film: accumulate in place.
-    DevBuf hsum, hsq;
     double *dsum, *dsq;
     if (sum) {
-        hsum.upload(sum, filmN, dev.stream);
-        if (sumsq) hsq.upload(sumsq, filmN, dev.stream);
-        dsum = hsum.as<double>();
-        dsq = sumsq ? hsq.as<double>() : nullptr;
+        if (fromZero) {
+            dev.hostSum.ensure(filmN * sizeof(double));
+            PG_CHECK(hipMemsetAsync(dev.hostSum.p, 0, filmN * sizeof(double), dev.stream));
+        } else {
+            dev.hostSum.upload(sum, filmN, dev.stream);
+        }
+        if (sumsq) dev.hostSq.upload(sumsq, filmN, dev.stream);
+        dsum = dev.hostSum.as<double>();
+        dsq = sumsq ? dev.hostSq.as<double>() : nullptr;
     } else {
         if (!dev.filmSum.p || dev.filmW != s.width || dev.filmH != s.height)
             throw std::runtime_error("resident film not reset for this resolution");
@@ -2616,9 +2628,9 @@ void RenderExImpl(Device &dev, const prgpu::SceneDescEx &sd, const prgpu::Render
     PG_CHECK(hipStreamSynchronize(dev.stream));
 }
 
-void SampleRadianceImpl(Device &dev, const prgpu::SceneDescEx &sd, const prgpu::RenderParamsEx &rp,
+void SampleRadianceImpl(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, const prgpu::RenderParamsEx &rp,
                         prgpu::SampleRecordEx *out) {
-    EnsurePTScene(dev, sd, nullptr);
+    EnsurePTScene(dev, geomKey, sd, nullptr);
     DevScene s = MakeDevScene(dev, sd, rp);
     const DevScene *ds = UploadDevScene(dev, s);
     const int sw = s.width + 2 * s.margin, sh = s.height + 2 * s.margin, npix = sw * sh;
@@ -2627,7 +2639,7 @@ void SampleRadianceImpl(Device &dev, const prgpu::SceneDescEx &sd, const prgpu::
     Params p = MakeParams(rp);
     p.guide = p.train = 0;  // per-sample records are the plain path tracer's
     TraceBatch(dev, s, ds, p, 1, npix, sw);
-    DevBuf rec;
+    DevBuf &rec = dev.records;
     rec.ensure(size_t(npix) * sizeof(prgpu::SampleRecordEx));
     Bufs b = MakeBufs(pt);
     hipLaunchKernelGGL(k_finish, dim3((npix + kBlock - 1) / kBlock), dim3(kBlock), 0, dev.stream, ds, p, b, npix,

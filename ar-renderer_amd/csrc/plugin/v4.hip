@@ -11,6 +11,7 @@
 #include "pt_host.h"
 
 #include <cstring>
+#include <memory>
 #include <stdexcept>
 #include <vector>
 
@@ -150,7 +151,7 @@ void RenderV4Impl(Device &dev, const prgpu::SceneDesc &sd, const prgpu::RenderPa
     V4Scene s;
     Export(sd, s);
     // The scene's own geometry: the traversal reads the device-resident BVH of these primitives.
-    EnsureGeometry(dev, sd.prims, sd.primCount);
+    const uint64_t geomKey = EnsureGeometry(dev, sd.prims, sd.primCount);
     prgpu::RenderParamsEx p{};
     p.spp = rp.spp;
     p.firstSample = rp.firstSample;
@@ -161,10 +162,10 @@ void RenderV4Impl(Device &dev, const prgpu::SceneDesc &sd, const prgpu::RenderPa
     p.russianRoulette = 1;
     p.lightSampler = prgpu::LightSamplerBVH;
     const size_t n = size_t(sd.camera.width) * size_t(sd.camera.height) * 3;
-    std::vector<double> sum(n, 0.0);
+    const std::unique_ptr<double[]> sum(new double[n]);
     // Coated and sheen materials: the caller's sheen albedo table when it passes one (the
     // reference host fills it from SheenBxDF::Albedo), else the same table built here.
-    RenderExImpl(dev, s.desc, p, sum.data(), nullptr, sd.sheenAlbedo);
+    RenderExImpl(dev, geomKey, s.desc, p, sum.get(), nullptr, true, sd.sheenAlbedo);
     for (size_t i = 0; i < n; ++i) outXYZ[i] += float(sum[i]);
 }
 
