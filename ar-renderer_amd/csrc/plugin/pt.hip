@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <numeric>
@@ -208,9 +209,10 @@ Box3 PrimBounds(const prgpu::Primitive &p) {
 #endif
 constexpr int kSurfaceWaves = PG_SURFACE_WAVES, kMaterialWaves = PG_MATERIAL_WAVES;
 
-// Bufs::counts: queue lengths (in one line) and the ray counters of the persistent traversals.
-constexpr int kFetchIntersect = 32, kFetchShadow = kFetchIntersect + kFeedInts, kCountsInts = kFetchShadow + kFeedInts,
-              kCountsBytes = kCountsInts * 4;
+// Bufs::counts: queue lengths (in one line) and the ray counters of the persistent traversals, in two
+// sets that bounces use in turn (see TraceBatch).
+constexpr int kFetchIntersect = 32, kFetchShadow = kFetchIntersect + kFeedInts, kSetInts = kFetchShadow + kFeedInts;
+constexpr int kCountIds = 12;  // queue lengths
 
 struct PTScene {
     DevBuf prims, mats, specs, knots, lights, lightArea, lnodes, leafOf, infinite, powerCdf, powerFunc, media, grid, sheen;
@@ -229,6 +231,8 @@ struct PTScene {
     DevBuf emit, qes;
     DevBuf sceneBuf;  // the DevScene the kernels read through a pointer
     DevBuf sq;  // the shadow queue
+    // Pinned: [0 .. kCountIds) queue lengths read back, then the 64-bit word a bounce publishes its path
+    // count in.
     int *countsHost = nullptr;
     DevBuf counts;
     // The captured bounce rounds (see TraceBatch) and the key of what they were captured with.
@@ -243,8 +247,6 @@ struct PTScene {
 Device::Device() = default;
 Device::~Device() {
     pt.reset();
-    for (hipEvent_t &e : pipeEvents)
-        if (e) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
 }
 void ReleasePT(Device &d) {
@@ -610,9 +612,9 @@ void EnsurePTScene(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, 
         pt->filterSigma = sigma;
         pt->filterNorm = float(1.0 / (s1 * s1));
     }
-    PG_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pt->countsHost), kCountsBytes, hipHostMallocDefault));
-    pt->counts.ensure(kCountsBytes);
-    PG_CHECK(hipMemsetAsync(pt->counts.p, 0, kCountsBytes, s));
+    PG_CHECK(hipHostMalloc(reinterpret_cast<void **>(&pt->countsHost), (kCountIds + 4) * sizeof(int),
+                           hipHostMallocMapped | hipHostMallocCoherent));
+    pt->counts.ensure(2 * kSetInts * sizeof(int));
     PG_CHECK(hipStreamSynchronize(s));
     dev.pt = std::move(pt);
     dev.ptKey = key;
@@ -753,8 +755,7 @@ struct Bufs {
     int *qr;     // the next queue sorted by that key, which the next bounce traces
     int *raySortTotals, *raySortCursor;
     int qcap;
-    int *counts;  // [0] queue A, [1] queue B, [2] and [11] shadow queues (alternating bounces when the
-                  // shadow rays are traced with the next bounce's closest hits), [3..5] plain
+    int *counts;  // this bounce's set: [0] next path queue, [2] shadow queue, [3..5] plain
                   // material queues, [6] medium scattering vertices, [9] emission queue, [10]
                   // coated / sheen material queue,
                   // then the ray counters of the traversal and of the shadow walk (kFeedInts each)
@@ -769,7 +770,8 @@ struct Bufs {
                         // the secondary wavelengths), depth and flags on arrival, primitive (-1: escaped)
     Field<float4, 2> qeLpdf;
     int *sq;        // shadow queue (path slots; the shadow records are indexed by slot)
-    int shadowIdx;  // index in counts of the shadow queue's length this bounce appends to
+    int *countsIn;  // the previous bounce's set: the paths and shadow rays this bounce traces; cleared by
+                    // the material stage for the next bounce
     const float4 *gout;
     float4 *trec;
     float *train;
@@ -863,16 +865,16 @@ __device__ __forceinline__ int *queue_ptr(const Bufs &b, int *next, int q) {
 // Index in Bufs::counts of material family q's queue length (the layered family's is 10, the
 // medium scattering vertices' 6).
 __device__ __host__ constexpr int mat_count_index(int q) { return q == 3 ? 10 : (q == 4 ? 6 : 3 + q); }
-__device__ __forceinline__ int *count_ptr(const Bufs &b, int *nextCount, int q) {
-    return q < QNext ? b.counts + mat_count_index(q) : (q == QNext ? nextCount : (q == QEmit ? b.counts + 9 : b.counts + b.shadowIdx));
+__device__ __forceinline__ int *count_ptr(const Bufs &b, int q) {
+    return q < QNext ? b.counts + mat_count_index(q) : (q == QNext ? b.counts : (q == QEmit ? b.counts + 9 : b.counts + 2));
 }
 
 // Reserves the tile's ranges (one atomic instruction) and scatters the staged entries.
-__device__ __forceinline__ void tile_flush(TileStage &t, const Bufs &b, int *next, int *nextCount) {
+__device__ __forceinline__ void tile_flush(TileStage &t, const Bufs &b, int *next) {
     __syncthreads();
     if (threadIdx.x < QIds) {
         const int q = int(threadIdx.x), c = t.cnt[q];
-        t.base[q] = c > 0 ? atomicAdd(count_ptr(b, nextCount, q), c) : 0;
+        t.base[q] = c > 0 ? atomicAdd(count_ptr(b, q), c) : 0;
         t.cnt[q] = 0;
     }
     __syncthreads();
@@ -907,13 +909,6 @@ __device__ __forceinline__ V2 get2(Pcg &r) {
     float a = r.uniform();
     float c = r.uniform();
     return {a, c};
-}
-
-// Start of a bounce: every queue length and fetch counter but the current path queue's is zeroed
-// (a kernel rather than a memset, so that the bounce can be captured in a graph).
-__global__ __launch_bounds__(64) void k_reset_counts(int *counts, int keep, int keep2) {
-    for (int i = int(threadIdx.x); i < kCountsInts; i += 64)
-        if (i != keep && i != keep2) counts[i] = 0;
 }
 
 // Camera samples (src/integrators/path.cpp:61-70, src/cameras/camera.cpp:36-48).
@@ -967,23 +962,46 @@ __global__ __launch_bounds__(kBlock) void k_camera(const DevScene *__restrict__ 
         for (int j = 0; j < kGuideRecords; ++j) b.trec[6 * j * size_t(b.qcap) + slot] = make_float4(0, 0, 0, 0);
 }
 
+// The counts as the first bounce finds them: it takes every path, all else is zero.
+__global__ __launch_bounds__(kBlock) void k_first_counts(Bufs b, int n) {
+    for (int i = int(threadIdx.x); i < kSetInts; i += kBlock) {
+        b.counts[i] = 0;
+        b.countsIn[i] = i == 0 ? n : 0;
+    }
+}
+
 // A closest hit as the path state holds it: distance, primitive (-1: a miss), barycentrics.
 __device__ __forceinline__ float4 closest_hit(const TravState &t) {
     return t.found() ? make_float4(t.tMax, __int_as_float(t.prim), t.b1, t.b2) : make_float4(0, __int_as_float(-1), 0, 0);
 }
 
+// Where a bounce publishes the paths that enter it: (tag << 32 | paths) into a word of coherent host
+// memory, as its first kernel starts. No word: not published.
+struct Publish {
+    unsigned long long *word;
+    uint32_t tag;
+};
+__device__ __forceinline__ void publish(const Publish &p, int paths) {
+    if (p.word && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(p.word, (static_cast<unsigned long long>(p.tag) << 32) | uint32_t(paths), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Closest hits of the queued paths (persistent, see trace_queue).
 template <bool kStats>
 __global__ __launch_bounds__(kTraceBlock) PG_WAVES(8) void k_intersect(const DevScene *__restrict__ sp, Bufs b, const int *queue,
-                                                           const int *count, int *fetch, unsigned long long *counters) {
+                                                           Publish pub, unsigned long long *counters) {
     const DevScene &s = *sp;
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
     TraceStats st;
     uint32_t rays = 0;
     int slot = 0;
+    const TraceCtx c = s.trace;  // before the store (see k_material_plain)
+    const int n = b.countsIn[0];
+    publish(pub, n);
     trace_queue<kStats>(
-        s.trace, *count, fetch, lds, tid, &st,
+        c, n, b.counts + kFetchIntersect, lds, tid, &st,
         [&](int i, DRay &r, TravState &t) {
             slot = queue[i];
             const float4 o = b.o[slot], d = b.d[slot];
@@ -1263,10 +1281,10 @@ __device__ __forceinline__ void surface_vertex(const DevScene &s, const Params &
 
 template <bool kMedia, bool kInterfaces>
 __global__ __launch_bounds__(kBlock) PG_WAVES(kSurfaceWaves) void k_surface(const DevScene *__restrict__ sp, Params p, Bufs b, const int *queue,
-                                                    const int *count, int *nextQueue, int *nextCount) {
+                                                    int *nextQueue) {
     __shared__ TileStage ts;
     const DevScene &s = *sp;
-    const int n = *count;
+    const int n = b.countsIn[0];
     tile_begin(ts);
     for (int t0 = int(blockIdx.x) * kTile; t0 < n; t0 += int(gridDim.x) * kTile) {
 #pragma unroll 1
@@ -1279,7 +1297,7 @@ __global__ __launch_bounds__(kBlock) PG_WAVES(kSurfaceWaves) void k_surface(cons
             }
             tile_stage(ts, j, slot, q1, q2, key);
         }
-        tile_flush(ts, b, nextQueue, nextCount);
+        tile_flush(ts, b, nextQueue);
     }
 }
 
@@ -1512,8 +1530,7 @@ __device__ __forceinline__ void phase_vertex(const DevScene &s, const Params &p,
 }
 
 template <int kType, bool kMedia, bool kGuided = false>
-__global__ __launch_bounds__(kBlock) PG_WAVES(kType == QLayered ? 0 : kMaterialWaves) void k_material(const DevScene *__restrict__ sp, Params p, Bufs b, int *nextQueue,
-                                                     int *nextCount) {
+__global__ __launch_bounds__(kBlock) PG_WAVES(kType == QLayered ? 0 : kMaterialWaves) void k_material(const DevScene *__restrict__ sp, Params p, Bufs b, int *nextQueue) {
     __shared__ TileStage ts;
     const DevScene &s = *sp;
     const int n = b.counts[mat_count_index(kType)];
@@ -1526,26 +1543,22 @@ __global__ __launch_bounds__(kBlock) PG_WAVES(kType == QLayered ? 0 : kMaterialW
             int slot = 0, q1 = -1, q2 = -1, key = 0;
             if (i < n) {
                 slot = queue[i];
-                if constexpr (kType == QPhase) phase_vertex(s, p, b, slot, &q1, &q2, &key);
-                else material_vertex<kType, kMedia, kGuided>(s, p, b, i, slot, &q1, &q2, &key);
+                material_vertex<kType, kMedia, kGuided>(s, p, b, i, slot, &q1, &q2, &key);
             }
             tile_stage(ts, j, slot, q1, q2, key);
         }
-        tile_flush(ts, b, nextQueue, nextCount);
+        tile_flush(ts, b, nextQueue);
     }
 }
 
 // The plain families (diffuse from family f0 on, conductor, dielectric and, in scenes with media,
 // the medium scattering vertices) in one launch over their queues laid end to end: in late
 // bounces, where each family holds a few thousand paths, separate launches cost a latency tail
-// each. A wave meets at most the boundaries between the queues.
-#ifndef PG_FUSED_MATERIAL
-#define PG_FUSED_MATERIAL 1
-#endif
-constexpr bool kFusedMaterial = PG_FUSED_MATERIAL != 0;
+// each. A wave meets at most the boundaries between the queues. The launch also clears the previous
+// bounce's counts, which the traversal and surface stages have read.
 template <bool kMedia>
 __global__ __launch_bounds__(kBlock) PG_WAVES(kMaterialWaves) void k_material_plain(const DevScene *__restrict__ sp, Params p, Bufs b,
-                                                                                 int *nextQueue, int *nextCount, int f0) {
+                                                                                 int *nextQueue, int f0) {
     __shared__ TileStage ts;
     const DevScene &s = *sp;
     const int nD = f0 <= QDiffuse ? b.counts[mat_count_index(QDiffuse)] : 0;
@@ -1576,8 +1589,12 @@ __global__ __launch_bounds__(kBlock) PG_WAVES(kMaterialWaves) void k_material_pl
             }
             tile_stage(ts, j, slot, q1, q2, key);
         }
-        tile_flush(ts, b, nextQueue, nextCount);
+        tile_flush(ts, b, nextQueue);
     }
+    // (Last: a store ahead of the scene's loads would make the compiler take their addresses for
+    // clobbered and read the scene through vector loads: gems' material stage 8.5 instead of 4.2 ms.)
+    if (blockIdx.x == 0)
+        for (int i = int(threadIdx.x); i < kSetInts; i += kBlock) b.countsIn[i] = 0;
 }
 
 // ---- the material queues sorted by material and medium ---------------------------------------
@@ -1757,23 +1774,21 @@ __device__ __forceinline__ void shadow_add(const Bufs &b, int slot, const SS &T,
 // as with a launch of their own and every sample's result is unchanged. The shadow rays follow the
 // closest rays in one run of items, so a bounce has one traversal tail instead of two; late bounces,
 // where a few thousand rays take the whole launch latency, cost half as much.
-constexpr int kShadowCountB = 11;  // the second shadow queue length (see Bufs::counts)
-__host__ __device__ constexpr int shadow_count_index(int curIdx) { return curIdx ? kShadowCountB : 2; }
-
 template <bool kStats>
 __global__ __launch_bounds__(kTraceBlock) PG_WAVES(8) void k_trace_bounce(const DevScene *__restrict__ sp, Bufs b,
-                                                                        const int *queue, const int *count,
-                                                                        const int *shadowCount, int *fetch,
+                                                                        const int *queue, Publish pub,
                                                                         unsigned long long *counters) {
     const DevScene &s = *sp;
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
-    const int n = *count, ns = *shadowCount;
+    const TraceCtx c = s.trace;  // before the store (see k_material_plain)
+    const int n = b.countsIn[0], ns = b.countsIn[2];
+    publish(pub, n);
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
     TraceStats st;
     uint32_t raysC = 0, raysS = 0;
     int slot = 0;
     trace_queue<kStats>(
-        s.trace, n + ns, fetch, lds, tid, &st,
+        c, n + ns, b.counts + kFetchIntersect, lds, tid, &st,
         [&](int i, DRay &r, TravState &t) {
             const bool shadow = i >= n;
             slot = shadow ? b.sq[i - n] : queue[i];
@@ -1806,8 +1821,7 @@ __global__ __launch_bounds__(kTraceBlock) PG_WAVES(8) void k_trace_bounce(const 
 // closest-hit query each), with the media's transmittance along the way. Persistent: a finished
 // query's lane goes on to its record's next segment or to another record.
 template <bool kStats, bool kMedia, bool kInterfaces>
-__global__ __launch_bounds__(kTraceBlock) void k_shadow(const DevScene *__restrict__ sp, Bufs b, const int *count,
-                                                        int *fetch, unsigned long long *counters) {
+__global__ __launch_bounds__(kTraceBlock) void k_shadow(const DevScene *__restrict__ sp, Bufs b, unsigned long long *counters) {
     const DevScene &s = *sp;
     __shared__ uint32_t lds[kStackLds * kTraceBlock];
     const int tid = int(blockIdx.x * blockDim.x + threadIdx.x);
@@ -1816,7 +1830,7 @@ __global__ __launch_bounds__(kTraceBlock) void k_shadow(const DevScene *__restri
     int slot = 0, medium = -1, iter = 0;
     SS T(1.f);
     trace_queue<kStats>(
-        s.trace, *count, fetch, lds, tid, &st,
+        s.trace, b.counts[2], b.counts + kFetchShadow, lds, tid, &st,
         [&](int i, DRay &r, TravState &t) {
             slot = b.sq[i];
             const float4 so = b.so[slot], sd = b.sd[slot];
@@ -2158,7 +2172,7 @@ Bufs MakeBufs(PTScene &pt) {
     b.so.p = pt.shadow.as<float4>(); b.sd.p = b.so.p + 1; b.sc.p = b.so.p + 2; b.sp.p = b.so.p + 3;
     b.sn = pt.shadowN.as<float4>();
     b.qe.p = pt.emit.as<int4>(); b.qeLpdf.p = pt.emit.as<float4>() + 1;
-    b.q0 = pt.q0.as<int>(); b.q1 = pt.q1.as<int>(); b.counts = pt.counts.as<int>();
+    b.q0 = pt.q0.as<int>(); b.q1 = pt.q1.as<int>(); b.counts = pt.counts.as<int>(); b.countsIn = b.counts + kSetInts;
     b.qm = pt.qm.as<int>();
     b.qk = nullptr;  // set by a batch that sorts the material queues
     b.qms = pt.qms.as<int>();
@@ -2170,7 +2184,6 @@ Bufs MakeBufs(PTScene &pt) {
     b.raySortCursor = b.raySortTotals + kRaySortBins;
     b.qes = pt.qes.as<int>();
     b.sq = pt.sq.as<int>();
-    b.shadowIdx = 2;
     b.qcap = int(pt.cap);
     b.pfilm = pt.pfilm.as<float2>(); b.xyz = pt.xyz.as<float4>();
     b.gout = nullptr;
@@ -2287,6 +2300,33 @@ uint64_t BounceKey(const Params &p, const Bufs &b, const DevScene *ds, int tgrid
     return h;
 }
 
+// The path count published under `tag`. Ends with the stream: a stream that has completed or failed
+// without publishing it is an error. The stream is asked only every two seconds: a query puts a
+// barrier into it (asked every 0.1 ms, the gems frame took 24.0 instead of 21 ms).
+int AwaitPublished(hipStream_t st, const unsigned long long *word, uint32_t tag) {
+    using Clock = std::chrono::steady_clock;
+    constexpr auto kPatience = std::chrono::seconds(2);
+    auto ask = Clock::now() + kPatience;
+    for (uint32_t spins = 1;; ++spins) {
+        const unsigned long long v = __atomic_load_n(word, __ATOMIC_RELAXED);
+        if (uint32_t(v >> 32) == tag) return int(uint32_t(v));
+        if (spins % 1024 == 0 && Clock::now() >= ask) {
+            const hipError_t e = hipStreamQuery(st);
+            const unsigned long long last = __atomic_load_n(word, __ATOMIC_RELAXED);
+            if (uint32_t(last >> 32) == tag) return int(uint32_t(last));
+            if (e != hipErrorNotReady) {
+                PG_CHECK(e);
+                throw std::runtime_error("internal error: a bounce did not publish its path count");
+            }
+            (void)hipGetLastError();
+            ask = Clock::now() + kPatience;
+        }
+#if defined(__x86_64__) && !__HIP_DEVICE_COMPILE__
+        __builtin_ia32_pause();
+#endif
+    }
+}
+
 void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, int passes, int npix, int sw) {
     PTScene &pt = *dev.pt;
     hipStream_t st = dev.stream;
@@ -2303,19 +2343,19 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
     timer.Run(prgpu::KernCamera, n, nullptr, [&] {
         hipLaunchKernelGGL(k_camera, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, ds, p, b, n, npix, sw);
     });
+    hipLaunchKernelGGL(k_first_counts, dim3(1), dim3(kBlock), 0, st, b, n);
     PG_CHECK(hipGetLastError());
     int active = n;
-    hipLaunchKernelGGL(k_reset_counts, dim3(1), dim3(64), 0, st, b.counts, -1, -1);
-    pt.countsHost[0] = n;
-    PG_CHECK(hipMemcpyAsync(b.counts, pt.countsHost, sizeof(int), hipMemcpyHostToDevice, st));
     const int shadeGrid = std::max(1, std::min((active + kTile - 1) / kTile, dev.cus * dev.tune.shadeBlocksPerCU));
     // One bounce: closest hits of the current queue, the surface and emission stages, the
     // material families (which fill the next queue), the shadow rays. Every kernel reads its
     // queue length from device memory, so rounds can be queued without reading them back.
     // Without media or interfaces a bounce's shadow rays are traced in the next bounce's traversal
-    // launch (k_trace_bounce): a bounce appends them to shadow queue shadow_count_index(curIdx) and
-    // the next one, whose curIdx is the other, consumes them. After the last bounce a round over the
-    // empty path queue traces the last shadow rays.
+    // launch (k_trace_bounce). After the last bounce a round over the empty path queue traces the last
+    // shadow rays.
+    // Bounces use the two sets of counts in turn: a bounce reads the paths and shadow rays that enter
+    // it from the other set, appends to its own, and clears the other in the material stage, when its
+    // readers are done. So a round has no launch that only resets or copies counts (about 5 us each).
     const bool fused = !media && !interfaces;
     const bool sorted = dev.tune.materialSort != 0 && pt.sortable != 0;
     if (sorted) b.qk = pt.qk.as<int>();
@@ -2325,33 +2365,22 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
     if (raySorted) b.nk = pt.nk.as<int>();
     const int sortGrid = std::max(1, std::min(shadeGrid, dev.cus * 4));
     int pendingShadow = 0;  // shadow rays the next round traces (profiled rounds: read back)
-    auto round = [&](int curIdx, int bounce, int tgrid, int grid) {
-        const int nxtIdx = 1 - curIdx;
+    auto round = [&](int curIdx, int bounce, int tgrid, int grid, Publish pub) {
         int *cur = raySorted && bounce > 0 ? b.qr : (curIdx ? b.q1 : b.q0), *nxt = curIdx ? b.q0 : b.q1;
         Bufs rb = b;
-        const int sIn = shadow_count_index(1 - curIdx);
-        rb.shadowIdx = fused ? shadow_count_index(curIdx) : 2;
-        hipLaunchKernelGGL(k_reset_counts, dim3(1), dim3(64), 0, st, b.counts, curIdx, fused ? sIn : -1);
+        rb.counts = b.counts + curIdx * kSetInts;
+        rb.countsIn = b.counts + (1 - curIdx) * kSetInts;
         timer.Run(prgpu::KernIntersect, int64_t(active) + (fused ? pendingShadow : 0), nullptr, [&] {
-            if (fused) {
-                auto *k = stats ? k_trace_bounce<true> : k_trace_bounce<false>;
-                hipLaunchKernelGGL(k, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, cur, b.counts + curIdx, b.counts + sIn,
-                                   b.counts + kFetchIntersect, ctr);
-            } else if (stats) {
-                hipLaunchKernelGGL(k_intersect<true>, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, cur, b.counts + curIdx,
-                                   b.counts + kFetchIntersect, ctr);
-            } else {
-                hipLaunchKernelGGL(k_intersect<false>, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, cur, b.counts + curIdx,
-                                   b.counts + kFetchIntersect, ctr);
-            }
+            auto *k = fused ? (stats ? k_trace_bounce<true> : k_trace_bounce<false>)
+                            : (stats ? k_intersect<true> : k_intersect<false>);
+            hipLaunchKernelGGL(k, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, cur, pub, ctr);
         });
         // Guiding applies to the vertices of the first guideBounces bounces (0: all).
         const bool guided = p.guide && (dev.tune.guideBounces == 0 || bounce < dev.tune.guideBounces);
         timer.Run(prgpu::KernSurface, active, nullptr, [&] {
             auto *k = media ? (interfaces ? k_surface<true, true> : k_surface<true, false>)
                             : (interfaces ? k_surface<false, true> : k_surface<false, false>);
-            hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), 0, st, ds, p, rb, cur, b.counts + curIdx, nxt,
-                               b.counts + nxtIdx);
+            hipLaunchKernelGGL(k, dim3(grid), dim3(kBlock), 0, st, ds, p, rb, cur, nxt);
             if (s.emitters) hipLaunchKernelGGL(k_emit, dim3(grid), dim3(kBlock), 0, st, ds, rb);
             if (sorted) {
                 hipLaunchKernelGGL(k_sort_count, dim3(sortGrid), dim3(kBlock), 0, st, rb);
@@ -2364,36 +2393,24 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
         if (sorted) mb.qm = b.qms;
         if (guided)
             timer.Run(prgpu::KernGuide, 0, nullptr, [&] {
-                dev.guide->Infer(mb.qm + size_t(QDiffuse) * b.qcap, b.counts + mat_count_index(QDiffuse), active, b.h0.p,
+                dev.guide->Infer(mb.qm + size_t(QDiffuse) * b.qcap, rb.counts + mat_count_index(QDiffuse), active, b.h0.p,
                                  b.h1.p, b.d.p, p.box, dev.cus, st);
             });
         timer.Run(prgpu::KernMaterial, active, nullptr, [&] {
             if (guided) {
                 auto *kd = media ? k_material<QDiffuse, true, true> : k_material<QDiffuse, false, true>;
-                hipLaunchKernelGGL(kd, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx);
+                hipLaunchKernelGGL(kd, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt);
             }
-            if (kFusedMaterial) {
-                auto *kp = media ? k_material_plain<true> : k_material_plain<false>;
-                hipLaunchKernelGGL(kp, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx,
-                                   guided ? int(QConductor) : int(QDiffuse));
-            } else {
-                auto *kd = media ? k_material<QDiffuse, true> : k_material<QDiffuse, false>;
-                auto *kc = media ? k_material<QConductor, true> : k_material<QConductor, false>;
-                auto *ke = media ? k_material<QDielectric, true> : k_material<QDielectric, false>;
-                if (!guided) hipLaunchKernelGGL(kd, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx);
-                hipLaunchKernelGGL(kc, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx);
-                hipLaunchKernelGGL(ke, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx);
-                auto *kph = k_material<QPhase, true>;
-                if (media) hipLaunchKernelGGL(kph, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx);
-            }
+            auto *kp = media ? k_material_plain<true> : k_material_plain<false>;
+            hipLaunchKernelGGL(kp, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, guided ? int(QConductor) : int(QDiffuse));
             if (pt.hasLayered) {
                 auto *kl = media ? k_material<QLayered, true> : k_material<QLayered, false>;
-                hipLaunchKernelGGL(kl, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt, b.counts + nxtIdx);
+                hipLaunchKernelGGL(kl, dim3(grid), dim3(kBlock), 0, st, ds, p, mb, nxt);
             }
             if (raySorted) {  // the next bounce traces the queue sorted by ray key
-                hipLaunchKernelGGL(k_ray_sort_count, dim3(sortGrid), dim3(kBlock), 0, st, rb, b.counts + nxtIdx);
+                hipLaunchKernelGGL(k_ray_sort_count, dim3(sortGrid), dim3(kBlock), 0, st, rb, rb.counts);
                 hipLaunchKernelGGL(k_ray_sort_scan, dim3(1), dim3(kBlock), 0, st, rb);
-                hipLaunchKernelGGL(k_ray_sort_scatter, dim3(sortGrid), dim3(kBlock), 0, st, rb, b.counts + nxtIdx, nxt);
+                hipLaunchKernelGGL(k_ray_sort_scatter, dim3(sortGrid), dim3(kBlock), 0, st, rb, rb.counts, nxt);
             }
         });
         if (!fused)
@@ -2402,8 +2419,7 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
                                          : k_shadow<true, false, true>)
                                 : (media ? (interfaces ? k_shadow<false, true, true> : k_shadow<false, true, false>)
                                          : k_shadow<false, false, true>);
-                hipLaunchKernelGGL(k, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, b.counts + 2, b.counts + kFetchShadow,
-                                   ctr);
+                hipLaunchKernelGGL(k, dim3(tgrid), dim3(kTraceBlock), 0, st, ds, rb, ctr);
             });
     };
 
@@ -2421,7 +2437,7 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
             hipGraph_t g = nullptr;
             PG_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
-                for (int k = 0; k < graphRounds; ++k) round(k & 1, k, tgrid, shadeGrid);
+                for (int k = 0; k < graphRounds; ++k) round(k & 1, k, tgrid, shadeGrid, Publish{});
             } catch (...) {
                 (void)hipStreamEndCapture(st, &g);
                 if (g) (void)hipGraphDestroy(g);
@@ -2435,37 +2451,31 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
         }
         while (active > 0) {
             PG_CHECK(hipGraphLaunch(pt.bounceExec, st));
-            PG_CHECK(hipMemcpyAsync(pt.countsHost, b.counts, sizeof(int), hipMemcpyDeviceToHost, st));
+            PG_CHECK(hipMemcpyAsync(pt.countsHost, b.counts + kSetInts, sizeof(int), hipMemcpyDeviceToHost, st));
             PG_CHECK(hipStreamSynchronize(st));
             active = pt.countsHost[0];
         }
-        if (fused) round(0, graphRounds, tgrid, 1);  // the last replay's shadow rays
+        if (fused) round(0, graphRounds, tgrid, 1, Publish{});  // the last replay's shadow rays
     } else if (!dev.profileMode) {
         // Pipelined: round k + 1 is queued before the host waits for the path count of round k,
         // so the device never idles on a read-back. A round's grids are sized by the count the host
         // last saw, an upper bound (paths only ever leave the queues); the kernels read the exact
-        // count on the device. The count of the paths entering round k + 1 is copied right after
-        // round k, before round k + 2 could clear it.
-        int *slot = pt.countsHost + 8;  // two read-back slots, alternating
-        for (hipEvent_t &e : dev.pipeEvents)
-            if (!e) PG_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        hipEvent_t ready[2] = {dev.pipeEvents[0], dev.pipeEvents[1]};
+        // count on the device. A round publishes the paths that enter it as its traversal starts.
+        auto *word = reinterpret_cast<unsigned long long *>(pt.countsHost + kCountIds);
+        __atomic_store_n(word, 0ull, __ATOMIC_RELAXED);  // tags start at 1; nothing queued writes it
         int bound = n, curIdx = 0, k = 0;
         // With fused shadow rays a round's traversal also takes the previous round's shadow rays,
         // at most one per path that entered it (<= bnd as well).
         auto launch = [&](int r, int curI, int bnd) {
             round(curI, r, TraceGrid(dev, int64_t(bnd) * (fused && r > 0 ? 2 : 1)),
-                  std::max(1, std::min((bnd + kTile - 1) / kTile, shadeGrid)));
-            PG_CHECK(hipMemcpyAsync(slot + (r & 1), b.counts + (1 - curI), sizeof(int), hipMemcpyDeviceToHost, st));
-            PG_CHECK(hipEventRecord(ready[r & 1], st));
+                  std::max(1, std::min((bnd + kTile - 1) / kTile, shadeGrid)), Publish{word, uint32_t(r) + 1});
+            PG_CHECK(hipGetLastError());
         };
         launch(0, 0, bound);
         while (true) {
             // Round k is queued and bounds round k + 1 (bound >= paths entering round k >= those entering k + 1).
             launch(k + 1, 1 - curIdx, bound);
-            PG_CHECK(hipGetLastError());
-            PG_CHECK(hipEventSynchronize(ready[k & 1]));
-            bound = slot[k & 1];  // paths entering round k + 1
+            bound = AwaitPublished(st, word, uint32_t(k + 1) + 1);  // paths entering round k + 1
             curIdx = 1 - curIdx;
             ++k;
             if (bound == 0) break;  // round k (queued, empty) is the last
@@ -2477,14 +2487,15 @@ void TraceBatch(Device &dev, const DevScene &s, const DevScene *ds, Params p, in
         while (active > 0 || pendingShadow > 0) {
             const int tgrid = TraceGrid(dev, int64_t(active) + pendingShadow);
             const int grid = std::max(1, std::min((active + kTile - 1) / kTile, shadeGrid));
-            round(curIdx, bounce, tgrid, grid);
+            round(curIdx, bounce, tgrid, grid, Publish{});
             PG_CHECK(hipGetLastError());
-            PG_CHECK(hipMemcpyAsync(pt.countsHost, b.counts, (kShadowCountB + 1) * sizeof(int), hipMemcpyDeviceToHost, st));
+            PG_CHECK(hipMemcpyAsync(pt.countsHost, b.counts + curIdx * kSetInts, kCountIds * sizeof(int),
+                                    hipMemcpyDeviceToHost, st));
             PG_CHECK(hipStreamSynchronize(st));
             timer.Collect();
-            pendingShadow = fused ? pt.countsHost[shadow_count_index(curIdx)] : 0;
+            pendingShadow = fused ? pt.countsHost[2] : 0;
             curIdx = 1 - curIdx;
-            active = pt.countsHost[curIdx];
+            active = pt.countsHost[0];
             ++bounce;
         }
     }
