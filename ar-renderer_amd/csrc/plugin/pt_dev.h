@@ -67,8 +67,72 @@ PG_HD Lambda sample_visible(float u) {  // src/core/spectrum.cpp:11-41
     return w;
 }
 
+// f of each wavelength, one after the other: one copy of its code.
+template <class F> PG_HD SS spec_each(const Lambda &w, F f) {
+    float a = w.l[0], b = w.l[1], c = w.l[2], d = w.l[3];
+    SS r;
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k) {
+        const float v = f(a);
+        a = b;
+        b = c;
+        c = d;
+        r.v[0] = r.v[1];
+        r.v[1] = r.v[2];
+        r.v[2] = r.v[3];
+        r.v[3] = v;
+    }
+    return r;
+}
+
+// A piecewise-linear spectrum at four wavelengths (spec_base's values): the four interval searches
+// run in step, so that a step's four loads are in flight together. A search that has ended keeps its
+// interval. Every index stays within the table, also outside of its range and for NaN.
+PG_HD SS spec_piecewise(const float *L, int n, const Lambda &w) {
+    const float *V = L + n;
+    if (n < 2) return SS(n == 1 ? V[0] : 0.f);
+    const float lo = L[0], hi = L[n - 1], vLo = V[0], vHi = V[n - 1];
+    int first[4] = {1, 1, 1, 1}, len[4] = {n - 2, n - 2, n - 2, n - 2};
+    while ((len[0] | len[1] | len[2] | len[3]) > 0) {  // none is negative
+        for (int k = 0; k < 4; ++k) {
+            const int half = len[k] >> 1, mid = first[k] + half;
+            const bool r = len[k] > 0 && L[mid] <= w.l[k];
+            first[k] = r ? mid + 1 : first[k];
+            len[k] = r ? len[k] - (half + 1) : half;
+        }
+    }
+    SS out;
+    for (int k = 0; k < 4; ++k) {
+        const int o = clampi(first[k] - 1, 0, n - 2);
+        const float l = w.l[k], x = L[o], t = (l - x) / (L[o + 1] - x);
+        const float v = lerp(t, V[o], V[o + 1]);
+        out.v[k] = l <= lo ? vLo : (l >= hi ? vHi : v);
+    }
+    return out;
+}
+
+// spec_eval at the path's four wavelengths, the same values. One switch for the four: the shading
+// kernels wait for loads and for their own instructions (a spectrum is read at a dozen places of
+// each), so that the searches' loads overlap and the rarer kinds have their code once. With one
+// spectrum read per sampled light and medium, the plain material kernel has 47.6 k instead of 82.2 k
+// instructions, the surface kernel with media 10.0 k instead of 17.9 k: fog studio 26.3 -> 24.2 ms
+// (its material stage 12.7 -> 10.7 ms), cloud 17.5 -> 17.0 ms.
 PG_HD SS spec_sample(const SpecTable &t, int id, const Lambda &w) {
-    return {spec_eval(t, id, w.l[0]), spec_eval(t, id, w.l[1]), spec_eval(t, id, w.l[2]), spec_eval(t, id, w.l[3])};
+    if (id < 0) return SS(0.f);
+    const prgpu::SpectrumEx &s = t.s[id];
+    SS b;
+    switch (s.kind) {
+    case prgpu::SpecConstant: b = SS(s.p[0]); break;
+    case prgpu::SpecPiecewise: b = spec_piecewise(t.knots + s.offset, s.count, w); break;
+    case prgpu::SpecSigmoid:
+    case prgpu::SpecCauchy:
+    case prgpu::SpecTable95:
+        b = {spec_base(s, t.knots, w.l[0]), spec_base(s, t.knots, w.l[1]), spec_base(s, t.knots, w.l[2]),
+             spec_base(s, t.knots, w.l[3])};
+        break;
+    default: b = spec_each(w, [&](float l) { return spec_base(s, t.knots, l); }); break;
+    }
+    return s.scale == 1.f ? b : b * s.scale;
 }
 
 // ---- sampling warps (src/core/sampling.h) ------------------------------------------------------
@@ -1248,11 +1312,11 @@ PG_HD float shape_pdf_from(const prgpu::Primitive &pr, float area, V3 ref, V3 wi
 }
 
 // ---- lights (src/lights/light.cpp, sky.cpp:52-60, light_bvh.cpp:179-234) ---------------------------
+PG_HD float area_profile(const prgpu::LightEx &L, float c) { return L.cosPower > 0 ? powf(fabsf(c), L.cosPower) : 1.f; }
 PG_HD SS area_L(const DevScene &s, const prgpu::LightEx &L, V3 n, V3 w, const Lambda &lam) {
     float c = dot(n, w);
     if (!L.twoSided && c <= 0) return SS(0.f);
-    float prof = L.cosPower > 0 ? powf(fabsf(c), L.cosPower) : 1.f;
-    return spec_sample(s.spec, L.spectrum, lam) * (L.scale * prof);
+    return spec_sample(s.spec, L.spectrum, lam) * (L.scale * area_profile(L, c));
 }
 
 struct LightSample {
@@ -1290,57 +1354,6 @@ PG_HD SS env_L(const DevScene &s, const prgpu::LightEx &L, V3 w, const Lambda &l
 
 PG_HD bool sample_li(const DevScene &s, int li, V3 p, V2 u, const Lambda &lam, LightSample *ls) {
     const prgpu::LightEx &L = s.lights[li];
-    if (L.kind == prgpu::LightExArea) {
-        const prgpu::Primitive &pr = s.prims[L.primitive];
-        ShapeSample ss;
-        if (!shape_sample_from(pr, s.lightArea[li], p, u, &ss) || ss.pdf == 0 || len2(ss.p - p) == 0) return false;
-        V3 wi = normalize(ss.p - p);
-        SS Le = area_L(s, L, ss.n, -wi, lam);
-        if (!Le.nonzero()) return false;
-        *ls = {Le, wi, ss.pdf, ss.p, ss.n};
-        return true;
-    }
-    if (L.kind == prgpu::LightExPoint) {
-        V3 d = f3(L.position) - p;
-        float d2 = len2(d);
-        if (d2 == 0) return false;
-        *ls = {spec_sample(s.spec, L.spectrum, lam) * (L.scale / d2), d / sqrtf(d2), 1, f3(L.position), V3()};
-        return true;
-    }
-    if (L.kind == prgpu::LightExSpot) {  // light.cpp:168-192
-        V3 d = f3(L.position) - p;
-        float d2 = len2(d);
-        if (d2 == 0) return false;
-        V3 wi = d / sqrtf(d2);
-        float f = smooth_step(dot(-wi, f3(L.direction)), L.cosFalloffEnd, L.cosFalloffStart);
-        if (f == 0) return false;
-        *ls = {spec_sample(s.spec, L.spectrum, lam) * (L.scale * f / d2), wi, 1, f3(L.position), V3()};
-        return true;
-    }
-    if (L.kind == prgpu::LightExGoniometric) {  // sky.cpp:12-27
-        V3 d = f3(L.position) - p;
-        float d2 = len2(d);
-        if (d2 == 0) return false;
-        V3 wi = d / sqrtf(d2);
-        float prof = ies_eval(s.spec.knots + L.profileOffset, -wi.x, -wi.y, -wi.z);
-        if (prof <= 0) return false;
-        *ls = {spec_sample(s.spec, L.spectrum, lam) * (L.scale * prof / d2), wi, 1, f3(L.position), V3()};
-        return true;
-    }
-    if (L.kind == prgpu::LightExSun) {  // sky.cpp:97-105
-        float cosMax = L.cosFalloffEnd;
-        float cosT = (1 - u.x) + u.x * cosMax;  // SampleUniformCone (sampling.h:47-53)
-        V3 wl = spherical_dir(safe_sqrt(1 - cosT * cosT), cosT, u.y * 2 * kPi);
-        V3 wi = Frame::from_z(f3(L.direction)).from_local(wl);
-        *ls = {spec_sample(s.spec, L.spectrum, lam) * L.scale, wi, 1 / (2 * kPi * (1 - cosMax)),
-               p + wi * (2 * s.worldR), V3()};
-        return true;
-    }
-    if (L.kind == prgpu::LightExDistant) {
-        V3 w = f3(L.direction);
-        *ls = {spec_sample(s.spec, L.spectrum, lam) * L.scale, w, 1, p + w * (2 * s.worldR), V3()};
-        return true;
-    }
     if (env_is_image(L)) {  // EnvironmentLight::SampleLi (src/lights/light.cpp:267-289)
         const EnvMap e = env_map(s.spec.knots + L.profileOffset);
         float mu, mv, mapPdf;
@@ -1352,8 +1365,54 @@ PG_HD bool sample_li(const DevScene &s, int li, V3 p, V2 u, const Lambda &lam, L
         *ls = {env_image_L(s, L, wi, lam), wi, mapPdf / (2 * kPi * kPi * sinTheta), p + wi * (2 * s.worldR), V3()};
         return true;
     }
-    V3 wi = uniform_sphere(u);
-    *ls = {spec_sample(s.spec, L.spectrum, lam) * L.scale, wi, kInv4Pi, p + wi * (2 * s.worldR), V3()};
+    // The other kinds' radiance is the light's spectrum times a factor of the kind.
+    float scale = L.scale, pdf = 1;
+    V3 wi, pl, nl;
+    if (L.kind == prgpu::LightExArea) {
+        const prgpu::Primitive &pr = s.prims[L.primitive];
+        ShapeSample ss;
+        if (!shape_sample_from(pr, s.lightArea[li], p, u, &ss) || ss.pdf == 0 || len2(ss.p - p) == 0) return false;
+        wi = normalize(ss.p - p);
+        const float c = dot(ss.n, -wi);
+        if (!L.twoSided && c <= 0) return false;
+        scale = L.scale * area_profile(L, c);
+        pdf = ss.pdf;
+        pl = ss.p;
+        nl = ss.n;
+    } else if (L.kind == prgpu::LightExPoint || L.kind == prgpu::LightExSpot || L.kind == prgpu::LightExGoniometric) {
+        V3 d = f3(L.position) - p;
+        float d2 = len2(d);
+        if (d2 == 0) return false;
+        wi = d / sqrtf(d2);
+        pl = f3(L.position);
+        if (L.kind == prgpu::LightExSpot) {  // light.cpp:168-192
+            float f = smooth_step(dot(-wi, f3(L.direction)), L.cosFalloffEnd, L.cosFalloffStart);
+            if (f == 0) return false;
+            scale = L.scale * f;
+        } else if (L.kind == prgpu::LightExGoniometric) {  // sky.cpp:12-27
+            float prof = ies_eval(s.spec.knots + L.profileOffset, -wi.x, -wi.y, -wi.z);
+            if (prof <= 0) return false;
+            scale = L.scale * prof;
+        }
+        scale = scale / d2;
+    } else {
+        if (L.kind == prgpu::LightExSun) {  // sky.cpp:97-105
+            float cosMax = L.cosFalloffEnd;
+            float cosT = (1 - u.x) + u.x * cosMax;  // SampleUniformCone (sampling.h:47-53)
+            V3 wl = spherical_dir(safe_sqrt(1 - cosT * cosT), cosT, u.y * 2 * kPi);
+            wi = Frame::from_z(f3(L.direction)).from_local(wl);
+            pdf = 1 / (2 * kPi * (1 - cosMax));
+        } else if (L.kind == prgpu::LightExDistant) {
+            wi = f3(L.direction);
+        } else {
+            wi = uniform_sphere(u);
+            pdf = kInv4Pi;
+        }
+        pl = p + wi * (2 * s.worldR);
+    }
+    const SS Le = spec_sample(s.spec, L.spectrum, lam) * scale;
+    if (L.kind == prgpu::LightExArea && !Le.nonzero()) return false;
+    *ls = {Le, wi, pdf, pl, nl};
     return true;
 }
 
@@ -1518,18 +1577,21 @@ PG_HD float grid_density(const DevScene &s, const prgpu::MediumEx &m, V3 p) {
     return lerp(dz, lerp(dy, c00, c10), lerp(dy, c01, c11));
 }
 
+PG_HD SS homogeneous_tr(const SS &st, float tMax) {
+    if (is_inf(tMax)) return {st.v[0] > 0 ? 0.f : 1.f, st.v[1] > 0 ? 0.f : 1.f, st.v[2] > 0 ? 0.f : 1.f,
+                              st.v[3] > 0 ? 0.f : 1.f};
+    return ss_exp_neg(st, tMax);
+}
+
 PG_HD SS medium_tr(const DevScene &s, int mi, V3 ro, V3 rd, float tMax, const Lambda &lam) {
     const prgpu::MediumEx &m = s.media[mi];
-    if (m.kind == prgpu::MediumHomogeneous) {
-        SS st = spec_sample(s.spec, m.sigmaA, lam) * m.scale + spec_sample(s.spec, m.sigmaS, lam) * m.scale;
-        if (is_inf(tMax)) return {st.v[0] > 0 ? 0.f : 1.f, st.v[1] > 0 ? 0.f : 1.f, st.v[2] > 0 ? 0.f : 1.f,
-                                  st.v[3] > 0 ? 0.f : 1.f};
-        return ss_exp_neg(st, tMax);
-    }
+    const bool grid = m.kind != prgpu::MediumHomogeneous;
     V3 mo, md;
     float t0, t1;
-    if (!grid_clip(m, ro, rd, tMax, &mo, &md, &t0, &t1)) return SS(1.f);
-    SS st = (spec_sample(s.spec, m.sigmaA, lam) + spec_sample(s.spec, m.sigmaS, lam)) * m.scale;
+    if (grid && !grid_clip(m, ro, rd, tMax, &mo, &md, &t0, &t1)) return SS(1.f);
+    const SS sa = spec_sample(s.spec, m.sigmaA, lam), sc = spec_sample(s.spec, m.sigmaS, lam);
+    if (!grid) return homogeneous_tr(sa * m.scale + sc * m.scale, tMax);
+    SS st = (sa + sc) * m.scale;
     float mu = m.maxDensity * st.maxc();
     if (mu <= 0) return SS(1.f);
     uint64_t w1[3] = {fbits(ro.x, ro.y), fbits(ro.z, rd.x), fbits(rd.y, rd.z)};
@@ -1557,9 +1619,15 @@ PG_HD DistSample medium_sample(const DevScene &s, int mi, V3 ro, V3 rd, float tM
     DistSample ds;
     ds.scattered = false;
     ds.pdfRatio = SS(1.f);
-    if (m.kind == prgpu::MediumHomogeneous) {  // SampleDistanceHero (medium.cpp:71-103)
-        SS ss = spec_sample(s.spec, m.sigmaS, lam) * m.scale;
-        SS st = spec_sample(s.spec, m.sigmaA, lam) * m.scale + ss;
+    const bool grid = m.kind != prgpu::MediumHomogeneous;
+    ds.weight = SS(1.f);
+    ds.t = tMax;
+    V3 mo, md;
+    float t0, t1;
+    if (grid && !grid_clip(m, ro, rd, tMax, &mo, &md, &t0, &t1)) return ds;
+    const SS sa = spec_sample(s.spec, m.sigmaA, lam) * m.scale, ssc = spec_sample(s.spec, m.sigmaS, lam) * m.scale;
+    const SS st = sa + ssc;
+    if (!grid) {  // SampleDistanceHero (medium.cpp:71-103)
         float t = st.v[0] > 0 ? -log_f32(1 - minf(u, kOneMinusEps)) / st.v[0] : kInfF;
         if (t < tMax) {
             SS Tr = ss_exp_neg(st, t);
@@ -1570,12 +1638,11 @@ PG_HD DistSample medium_sample(const DevScene &s, int mi, V3 ro, V3 rd, float tM
                 ds.weight = SS(0.f);
                 return ds;
             }
-            ds.weight = Tr * ss / pdf0;
+            ds.weight = Tr * ssc / pdf0;
             ds.pdfRatio = st * Tr / pdf0;
             return ds;
         }
-        SS Tr = medium_tr(s, mi, ro, rd, tMax, lam);
-        ds.t = tMax;
+        SS Tr = homogeneous_tr(st, tMax);
         if (!(Tr.v[0] > 0)) {
             ds.weight = SS(0.f);
             return ds;
@@ -1585,13 +1652,6 @@ PG_HD DistSample medium_sample(const DevScene &s, int mi, V3 ro, V3 rd, float tM
         return ds;
     }
     // Grid: spectral tracking (medium.cpp:232-285).
-    ds.weight = SS(1.f);
-    ds.t = tMax;
-    V3 mo, md;
-    float t0, t1;
-    if (!grid_clip(m, ro, rd, tMax, &mo, &md, &t0, &t1)) return ds;
-    SS sa = spec_sample(s.spec, m.sigmaA, lam) * m.scale, ssc = spec_sample(s.spec, m.sigmaS, lam) * m.scale;
-    SS st = sa + ssc;
     float mu = m.maxDensity * st.maxc();
     if (mu <= 0) return ds;
     auto avg = [&](const SS &x) {

@@ -1,0 +1,93 @@
+"""spec_sample (pt_dev.h) evaluates a spectrum at four wavelengths with one switch and one search in
+step; spec_eval evaluates one. Compiled for the host, both must return the same bits for every kind
+that a scene can hold: constant, sigmoid, blackbody, Sellmeier, Cauchy, the 95-sample table, and
+piecewise tables of 0 to 130 knots, at wavelengths below, on, between and above the knots.
+"""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include "pt_dev.h"
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include <vector>
+using namespace pgpu;
+int main() {
+    std::mt19937 g(7);
+    std::uniform_real_distribution<float> u(0, 1);
+    std::vector<float> knots;
+    std::vector<prgpu::SpectrumEx> specs;
+    auto add = [&](int kind, int count, float scale) {
+        prgpu::SpectrumEx s{};
+        s.kind = decltype(s.kind)(kind);
+        s.scale = scale;
+        s.count = count;
+        s.offset = int(knots.size());
+        specs.push_back(s);
+        return &specs.back();
+    };
+    const int sizes[] = {0, 1, 2, 3, 4, 5, 7, 8, 9, 31, 64, 95, 130};
+    for (float scale : {1.f, 0.37f}) {
+        add(prgpu::SpecConstant, 0, scale)->p[0] = 0.3f;
+        auto *q = add(prgpu::SpecSigmoid, 0, scale);
+        q->p[0] = -3e-5f; q->p[1] = 0.03f; q->p[2] = -7.f;
+        q = add(prgpu::SpecBlackbody, 0, scale);
+        q->p[0] = 5600; q->p[1] = 1e-9f;
+        q = add(prgpu::SpecSellmeier, 3, scale);
+        const float bk7[6] = {1.0396f, 0.2318f, 1.0105f, 0.0060f, 0.0200f, 103.56f};
+        std::memcpy(q->p, bk7, sizeof bk7);
+        q = add(prgpu::SpecCauchy, 0, scale);
+        q->p[0] = 1.5f; q->p[1] = 4200;
+        add(prgpu::SpecTable95, prgpu::kSpectrumSamples, scale);
+        for (int i = 0; i < prgpu::kSpectrumSamples; ++i) knots.push_back(u(g));
+        for (int n : sizes) {
+            add(prgpu::SpecPiecewise, n, scale);
+            for (int i = 0; i < n; ++i) knots.push_back(400 + 350.f * (i + (i ? 0.5f * u(g) : 0.f)) / n);
+            for (int i = 0; i < n; ++i) knots.push_back(u(g));
+        }
+    }
+    const SpecTable t{specs.data(), knots.data()};
+    long bad = 0, checked = 0;
+    for (int id = -1; id < int(specs.size()); ++id)
+        for (int trial = 0; trial < 400; ++trial) {
+            Lambda w;
+            for (int k = 0; k < 4; ++k) {
+                w.l[k] = 360 + 470 * u(g);
+                w.pdf[k] = 1;
+                const bool table = id >= 0 && specs[id].kind == prgpu::SpecPiecewise && specs[id].count > 0;
+                if (table && trial % 2) w.l[k] = knots[specs[id].offset + int(u(g) * specs[id].count)];
+            }
+            const SS v = spec_sample(t, id, w);
+            for (int k = 0; k < 4; ++k, ++checked) {
+                const float e = spec_eval(t, id, w.l[k]);
+                if (std::memcmp(&e, &v.v[k], 4)) {
+                    if (bad++ < 5) std::printf("spectrum %d at %.9g: %.9g, not %.9g\n", id, w.l[k], v.v[k], e);
+                }
+            }
+        }
+    std::printf("%ld values, %ld differ\n", checked, bad);
+    return bad != 0;
+}
+"""
+
+
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+def test_four_wavelengths_equal_one_by_one(tmp_path):
+    (tmp_path / "t.hip").write_text(SOURCE)
+    exe = str(tmp_path / "t")
+    subprocess.run(
+        [HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-ffp-contract=off", "-w", "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "ar-renderer_amd", "csrc", "plugin"),
+         str(tmp_path / "t.hip"), "-o", exe],
+        check=True,
+    )
+    r = subprocess.run([exe], capture_output=True, text=True)
+    assert r.returncode == 0, r.stdout
