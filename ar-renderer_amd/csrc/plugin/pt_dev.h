@@ -1129,16 +1129,43 @@ PG_HD void dielectric_bx(const DevScene &s, const prgpu::Material &m, Lambda &la
 }
 
 // kFamily: -1 = any plain material, else the material family the caller guarantees (0 diffuse,
-// 1 conductor, 2 dielectric), which removes the other families' code from the caller.
+// 1 conductor, 2 dielectric), which removes the other families' code from the caller. The closure's
+// fields are joined in locals and written once: written through the branches, the record would stay
+// in scratch memory.
 template <int kFamily = -1>
 PG_HD BSDF eval_surface(const DevScene &s, const prgpu::Material &m, const Surf &si, Lambda &lam) {
+    int type;
+    float etaD = 1, ax = 0, ay = 0;
+    SS ba, bb;
+    if (kFamily == 0 || (kFamily < 0 && m.type == prgpu::MatDiffuse)) {
+        BxDF x;
+        diffuse_bx(s, m, si, lam, x);
+        type = x.type;
+        ba = x.a;
+    } else if (kFamily == 1 || (kFamily < 0 && m.type == prgpu::MatConductor)) {
+        BxDF x;
+        conductor_bx(s, m, si, lam, 0.f, x);
+        type = x.type;
+        ax = x.dist.ax;
+        ay = x.dist.ay;
+        ba = x.a;
+        bb = x.b;
+    } else {
+        BxDF x;
+        x.dist.ax = x.dist.ay = 0;
+        dielectric_bx(s, m, lam, x);
+        type = x.type;
+        etaD = x.etaD;
+        ax = x.dist.ax;
+        ay = x.dist.ay;
+    }
     BSDF b;
-    BxDF &bx = b.bx;
-    bx.etaD = 1;
-    bx.dist.ax = bx.dist.ay = 0;
-    if (kFamily == 0 || (kFamily < 0 && m.type == prgpu::MatDiffuse)) diffuse_bx(s, m, si, lam, bx);
-    else if (kFamily == 1 || (kFamily < 0 && m.type == prgpu::MatConductor)) conductor_bx(s, m, si, lam, 0.f, bx);
-    else dielectric_bx(s, m, lam, bx);
+    b.bx.type = type;
+    b.bx.etaD = etaD;
+    b.bx.dist.ax = ax;
+    b.bx.dist.ay = ay;
+    b.bx.a = ba;
+    b.bx.b = bb;
     b.frame = Frame::from_xz(si.dpdus, si.ns);
     return b;
 }
