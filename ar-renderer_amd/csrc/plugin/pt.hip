@@ -1,10 +1,11 @@
 // Wavefront spectral path tracer for gfx950.
 //
 // A batch holds P passes x (sample width x sample height) camera samples, one path slot each.
-// Per bounce: k_intersect (closest hit of every queued path), k_shade (one iteration of the
-// reference's Li loop: media, emission, interfaces, BSDF, next-event estimation, Russian
-// roulette; surviving paths are appended to the next queue, shadow rays to the shadow queue),
-// k_shadow (transmittance of the shadow rays; visible contributions are added to their path).
+// Per bounce: k_trace_bounce (closest hit of every queued path and the previous bounce's shadow rays;
+// in scenes with media or interfaces k_intersect, and k_shadow after the materials), k_surface (media,
+// interfaces, the hit's vertex record; paths are dealt to one queue per material family), k_emit
+// (emission met), k_material_plain and k_material (BSDF, next-event estimation, Russian roulette;
+// surviving paths are appended to the next queue, shadow rays to the shadow queue).
 // When the queue drains, k_finish turns each path's radiance into a film sample and k_gather
 // splats the samples of every pass onto the image with the film's reconstruction filter,
 // adding the pass value and its square to the FP64 sum and sum-of-squares accumulators.
@@ -196,10 +197,10 @@ Box3 PrimBounds(const prgpu::Primitive &p) {
 // Minimum waves per SIMD a kernel is compiled for (its register budget: 8 waves = 64 VGPRs,
 // 6 = 80, 5 = 96, 4 = 128, 3 = 168); 0 leaves the choice to the compiler. The traversal is
 // latency-bound and its LDS stacks allow 8 waves per SIMD, which 64 VGPRs reach without spilling.
-// The plain material families take 175-185 VGPRs unconstrained (2 waves); measured on
-// configuration 2 at 1920x1080, 4 spp: 5.13 ms per step at 2 waves, 4.69 at 3, 4.80 at 4 (the
-// spills of a 128-VGPR budget cost more than the occupancy gains). The surface stage is fastest
-// unconstrained (92 VGPRs: 1.61 ms; 1.71 at 6 waves, 2.23 at 8).
+// The plain material families take 174-190 VGPRs unconstrained (2 waves) and 168 at 3 waves without
+// spills in scenes without media; a 128-VGPR budget (4 waves) spills 26-28 registers and is slower:
+// terrain 62.2 -> 63.6 ms, cloud 17.0 -> 17.8, gems 19.3 -> 19.5. The surface stage (105-162 VGPRs)
+// and the emission stage (151) are left unconstrained.
 #define PG_WAVES(n) __attribute__((amdgpu_waves_per_eu((n) > 0 ? (n) : 1, 8)))
 #ifndef PG_SURFACE_WAVES
 #define PG_SURFACE_WAVES 0

@@ -40,12 +40,13 @@ def kernel_bytes(name, stats, items, fused=False):
     """Algorithmic HBM bytes of one kind of launch, from its item count and the traversal counters.
 
     intersect: per ray 32 B ray in (origin, direction) + 4 B queue entry + 16 B hit out, plus
-      128 B per wide node fetched and 48 B per leaf record tested.
-    shadow: per shadow ray 112 B record + 32 B wavelengths in, 32 B radiance read-modify-write,
-      plus the same node and record bytes.
-    surface: per path 80 B of path state and hit read, the 128 B primitive, 80 B written, 8 B
-      of queue entries. material: per path 176 B read, 112 B written, the 88 B material and a
-      112 B shadow record.
+      the bytes of the wide nodes fetched and of the leaf records tested.
+    shadow: per shadow ray a 48 B record in and 32 B radiance read-modify-write in the fused launch;
+      with media or interfaces 80 B record + 32 B wavelengths in and 64 B read-modify-write; plus the
+      same node and record bytes.
+    surface: per path the 64 B ray record read, the 128 B primitive, the 64 B vertex record written,
+      8 B of queue entries. material: per path 160 B read, 112 B written, the 88 B material and a
+      48 B shadow record.
     """
     nb, rb = stats["nodeBytes"], stats["recBytes"]
     if name == "intersect" and fused:
@@ -53,7 +54,7 @@ def kernel_bytes(name, stats, items, fused=False):
         # rays: its items are both, and the bytes per item their mix
         rc, rs = stats["closestRays"], stats["shadowRays"]
         per = ((52 * rc + nb * stats["closestNodes"] + rb * stats["closestRecs"]) +
-               (176 * rs + nb * stats["shadowNodes"] + rb * stats["shadowRecs"])) / max(1, rc + rs)
+               (80 * rs + nb * stats["shadowNodes"] + rb * stats["shadowRecs"])) / max(1, rc + rs)
         return per * items, per
     if name == "intersect":
         rays = max(1, stats["closestRays"])
@@ -64,14 +65,14 @@ def kernel_bytes(name, stats, items, fused=False):
         per = 176 + nb * stats["shadowNodes"] / rays + rb * stats["shadowRecs"] / rays
         return per * items, per
     if name == "surface":
-        # 80 B path state and hit in, the 128 B primitive, 64 B hit record and 16 B state out,
-        # 8 B of queue entries
-        per = 80 + 128 + 80 + 8
+        # the ray record (ray, hit, state) in, the 128 B primitive, the vertex record out, 8 B of
+        # queue entries
+        per = 64 + 128 + 64 + 8
         return per * items, per
     if name == "material":
-        # 176 B path state and hit record in, 112 B state out, the 88 B material, and a 112 B
+        # direction, state, path and vertex record in, 112 B state out, the 88 B material, and a 48 B
         # shadow record
-        per = 176 + 112 + 88 + 112
+        per = 160 + 112 + 88 + 48
         return per * items, per
     return None, None
 
