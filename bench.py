@@ -36,6 +36,9 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "trace_bounce_terrain_1080p_traffi
 METRIC = "Msamples/s and equal-time relMSE, guided vs plain PT, 1080p on one MI355X"
 
 
+NODE_READ = 80  # bytes of a wide node that the traversal loads; its line in memory has stats["nodeBytes"]
+
+
 def kernel_bytes(name, stats, items, fused=False):
     """Algorithmic HBM bytes of one kind of launch, from its item count and the traversal counters.
 
@@ -48,7 +51,7 @@ def kernel_bytes(name, stats, items, fused=False):
       8 B of queue entries. material: per path 160 B read, 112 B written, the 88 B material and a
       48 B shadow record.
     """
-    nb, rb = stats["nodeBytes"], stats["recBytes"]
+    nb, rb = NODE_READ, stats["recBytes"]
     if name == "intersect" and fused:
         # one launch per bounce traces the bounce's closest rays and the previous bounce's shadow
         # rays: its items are both, and the bytes per item their mix
@@ -345,12 +348,12 @@ def traversal_counts(pa, host, plugin):
         rows[name] = {
             "rays": int(n), "hit_rate": round(float((hits["prim"] >= 0).mean()), 4),
             "wide_bvh": {"nodes_per_ray": round(nodes, 3), "records_per_ray": round(recs, 3),
-                         "bytes_per_ray": round(nodes * st["nodeBytes"] + recs * st["recBytes"] + 52, 1)},
+                         "bytes_per_ray": round(nodes * NODE_READ + recs * st["recBytes"] + 52, 1)},
             "reference_bvh": {"nodes_per_ray": round(float(ref[0]), 3), "primitives_per_ray": round(float(ref[1]), 3),
                               "hit_rate": round(float(ref[2]), 4),
                               "bytes_per_ray": round(float(ref[0]) * 32 + float(ref[1]) * 128 + 48, 1)}}
     print(json.dumps({"traversal_counts": rows, "scene": "configuration 2 at 1920x1080",
-                      "bytes": "wide: 128 B node + 48 B record + 32 B ray + 4 B queue + 16 B hit; "
+                      "bytes": "wide: 80 B node + 48 B record + 32 B ray + 4 B queue + 16 B hit; "
                                "reference: 32 B node + 128 B primitive + 32 B ray + 16 B hit"}), flush=True)
 
 
@@ -510,14 +513,14 @@ def main():
             avg_ms = kernels[dominant]["ms"] / max(1, kernels[dominant]["launches"])
             # `frac` prices the algorithmic bytes (every node and record fetch counted as if it came
             # from HBM) against the HBM peak; `frac_hbm_traffic` prices the counter-measured HBM bytes
-            # of one launch. Most node and record re-reads hit L2 / MALL, so the kernel is limited by
-            # the latency of its dependent fetches, not by HBM bandwidth.
+            # of one launch. Most node and record re-reads hit L2 / MALL, and the SIMDs' issue slots are
+            # full (counters: VALU busy, 58 % of lanes active), so HBM bandwidth is not the limit.
             roofline = {"bound": "hbm", "kernel": dominant, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                         "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                         "traffic": traffic,
                         "frac_hbm_traffic": (round(traffic / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)
                                              if traffic else None),
-                        "limited_by": "latency of dependent node / record fetches (L2 / MALL hits)",
+                        "limited_by": "VALU issue at 58 % of lanes active; nodes and records come from L2 / MALL",
                         "algorithmic_bytes_per_item": round(per, 1),
                         "items_per_launch": round(kernels[dominant]["items"] / max(1, kernels[dominant]["launches"]), 1),
                         "avg_launch_ms": round(kernels[dominant]["ms"] / max(1, kernels[dominant]["launches"]), 4)}
