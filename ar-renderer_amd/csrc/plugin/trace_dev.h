@@ -171,12 +171,19 @@ __device__ __forceinline__ float slab_inv(float d) {
     return __builtin_copysignf(fminf(fabsf(r), 0x1p64f), d);
 }
 
+// The end of an unlimited ray. A plane distance that overflows is +inf: past this end, also once it is
+// widened (kSlabWiden), so a box at such a distance is not entered.
+constexpr float kTraceFar = 0x1.ffffp127f;
+
+// A ray whose origin is not finite, or whose range is empty or NaN, hits nothing and is complete at
+// once: the slab test's minima and maxima drop a NaN, so it would enter every node.
 __device__ __forceinline__ void trace_begin(TravState &t, const DRay &r, float tMax, bool any) {
     t.ix = slab_inv(r.dx);
     t.iy = slab_inv(r.dy);
     t.iz = slab_inv(r.dz);
-    t.tMax = tMax;
-    t.cur = 0;  // root node
+    t.tMax = fminf(tMax, kTraceFar);
+    const bool valid = __builtin_isfinite(r.ox) && __builtin_isfinite(r.oy) && __builtin_isfinite(r.oz) && tMax > 0.f;
+    t.cur = valid ? 0 : kIdle;  // the root node
     t.sp = 4 * int(threadIdx.x);
     t.any = any;
     t.prim = -1;
