@@ -209,8 +209,10 @@ __device__ __forceinline__ void trace_pop(const TraceCtx &c, TravState &t, uint3
 }
 
 // Conservative widening of the slab test (the reference's, bvh.cpp:137-156, on both ends), applied
-// to the exit distance alone: (1 + 6 eps) / (1 - 6 eps), rounded up. (To the distance, not to the
-// planes' coefficients: a flat box's entry and exit are then the same FMA and stay equal.)
+// to the far end alone, the lesser of the exit distance and the best hit: (1 + 6 eps) / (1 - 6 eps),
+// rounded up. The best hit's distance needs it as the exit does: a flat box's entry distance and its
+// triangle's hit distance are rounded separately. (To the distance, not to the planes' coefficients: a
+// flat box's entry and exit are then the same FMA and stay equal.)
 constexpr float kSlabWiden = 1.f + 1.6e-6f;
 
 // One wide node: slab-tests its children, pushes the hit ones far to near and continues with the
@@ -250,7 +252,7 @@ __device__ __forceinline__ void trace_node(const TraceCtx &c, const DRay &r, Tra
                                      __builtin_fmaf(float((nz[w] >> sh) & 0xff), az, cz)), 0.f);
         const float tf = fminf(fminf(fminf(__builtin_fmaf(float((fx[w] >> sh) & 0xff), ax, cx),
                                            __builtin_fmaf(float((fy[w] >> sh) & 0xff), ay, cy)),
-                                     __builtin_fmaf(float((fz[w] >> sh) & 0xff), az, cz)) * kSlabWiden, t.tMax);
+                                     __builtin_fmaf(float((fz[w] >> sh) & 0xff), az, cz)), t.tMax) * kSlabWiden;
         key[i] = tn <= tf ? ((__float_as_uint(tn) & ~7u) | uint32_t(i)) : 0xffffffffu;
     }
     sort8(key);
