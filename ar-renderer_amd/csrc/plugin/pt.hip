@@ -267,7 +267,9 @@ uint64_t PTKey(uint64_t geomKey, const prgpu::SceneDescEx &sd, const float *shee
     if (sd.knotCount) mix(sd.knots, sizeof(float) * size_t(sd.knotCount));
     if (sd.lightCount) mix(sd.lights, sizeof(prgpu::LightEx) * size_t(sd.lightCount));
     if (sd.mediumCount) mix(sd.media, sizeof(prgpu::MediumEx) * size_t(sd.mediumCount));
-    mix(&sd.gridCount, sizeof(sd.gridCount));
+    // The grid as GeometryKey takes the primitives: its address, and every step-th voxel.
+    const uint64_t grid[2] = {uint64_t(sd.gridCount), uint64_t(uintptr_t(sd.gridData))};
+    mix(grid, sizeof(grid));
     if (sd.gridCount > 0) {
         int64_t step = std::max<int64_t>(1, sd.gridCount / 4096);
         for (int64_t i = 0; i < sd.gridCount; i += step) mix(&sd.gridData[i], sizeof(float));

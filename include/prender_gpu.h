@@ -424,7 +424,10 @@ PRGPU_API int prgpu_tune_set(int deviceIndex, const char *key, double value);
 PRGPU_API int prgpu_tune_get(int deviceIndex, const char *key, double *value);
 // The tuning file read (0) or none (1), and the first invalid line found in it (empty if none).
 PRGPU_API int prgpu_tune_source(char *path, int pathLen, char *error, int errorLen);
-// Frees every device buffer the plugin holds for the device.
+// Frees every device buffer the plugin holds for the device. Also what a caller does after changing a
+// large array in place: a call takes a scene for the resident one when its counts, the addresses of the
+// primitives and the grid, every (count / 4096)-th primitive and voxel, the last primitive, and all of
+// the materials, spectra, knots, lights, media and camera are the same.
 PRGPU_API int prgpu_release(int deviceIndex);
 
 // ---- path-guiding model probes (no reference counterpart) ---------------------------------------

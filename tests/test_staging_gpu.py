@@ -2,7 +2,8 @@
 
 Host films, sample records and the guiding probes' arrays go through buffers kept from call to call:
 calls of changing size, with and without the sum of squares, must give what a first call gives. A
-scene changed in place, at the same addresses, must not be taken for the resident one.
+small scene, which the keys hash whole, changed in place, at the same addresses, must not be taken for the
+resident one (larger ones: test_residency_gpu.py).
 """
 import numpy as np
 import pytest
