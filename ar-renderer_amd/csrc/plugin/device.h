@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -46,6 +47,23 @@ struct DevBuf {
         ensure(count * sizeof(T));
         if (count) PG_CHECK(hipMemcpyAsync(p, src, count * sizeof(T), hipMemcpyHostToDevice, s));
     }
+};
+
+// Waits for the stream when its scope is left by an exception, so that nothing that a failed call has
+// queued runs beside a later call: a bounce's path count would be published under a tag that the later
+// call waits for, and copies would write arrays that the caller has got back.
+class DrainOnError {
+  public:
+    explicit DrainOnError(hipStream_t s) : stream(s), entered(std::uncaught_exceptions()) {}
+    DrainOnError(const DrainOnError &) = delete;
+    DrainOnError &operator=(const DrainOnError &) = delete;
+    ~DrainOnError() {
+        if (std::uncaught_exceptions() > entered) (void)hipStreamSynchronize(stream);
+    }
+
+  private:
+    hipStream_t stream;
+    int entered;
 };
 
 // Fingerprint of host data: 32 bytes a step in four independent lanes (xor, rotate, multiply: each

@@ -2473,7 +2473,9 @@ void TraceBatch(Device &dev, const DevScene &s, SceneArg ds, Params p, int passe
         // last saw, an upper bound (paths only ever leave the queues); the kernels read the exact
         // count on the device. A round publishes the paths that enter it as its traversal starts.
         auto *word = reinterpret_cast<unsigned long long *>(pt.countsHost + kCountIds);
-        __atomic_store_n(word, 0ull, __ATOMIC_RELAXED);  // tags start at 1; nothing queued writes it
+        // Tags start at 1. Nothing queued writes the word: the loop ends after the last round has
+        // published, and a failed call drains the stream (DrainOnError).
+        __atomic_store_n(word, 0ull, __ATOMIC_RELAXED);
         int bound = n, curIdx = 0, k = 0;
         // With fused shadow rays a round's traversal also takes the previous round's shadow rays,
         // at most one per path that entered it (<= bnd as well).
@@ -2530,6 +2532,7 @@ void RenderExImpl(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, c
         if (sum && fromZero) std::fill(sum, sum + filmN, 0.0);
         return;
     }
+    const DrainOnError drain(dev.stream);
     EnsurePTScene(dev, geomKey, sd, sheenTable);
     DevScene s = MakeDevScene(dev, sd, rp);
     const SceneArg ds = UploadDevScene(dev, s);
@@ -2652,6 +2655,7 @@ void RenderExImpl(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, c
 
 void SampleRadianceImpl(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, const prgpu::RenderParamsEx &rp,
                         prgpu::SampleRecordEx *out) {
+    const DrainOnError drain(dev.stream);
     EnsurePTScene(dev, geomKey, sd, nullptr);
     DevScene s = MakeDevScene(dev, sd, rp);
     const SceneArg ds = UploadDevScene(dev, s);

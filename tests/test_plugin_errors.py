@@ -1,0 +1,79 @@
+"""The plugin's host code after a failed launch or allocation, on the CPU: its sources compiled for the
+host alone run on a stand-in HIP runtime (tests/fake_hip/fake_hip.cpp) whose launches and allocations can
+be made to fail and whose stream can be watched. What a failed call leaves must not reach the next one.
+"""
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import pytest
+
+import prender_amd as pa
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+SRC = os.path.join(ROOT, "ar-renderer_amd", "csrc", "plugin")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = tmp_path_factory.mktemp("fake_hip")
+    inc = ["-I" + os.path.join(ROOT, "include"), "-I" + SRC, "-I/opt/rocm/include"]
+    jobs, objs = [], []
+    for name in ("api.hip", "pt.hip", "v4.hip", "guide.hip"):
+        objs.append(str(out / (name + ".o")))
+        jobs.append([HIPCC, "-x", "hip", "--offload-host-only", "--offload-arch=gfx950", "-fuse-cuid=none", "-std=c++17",
+                     "-O1", "-fPIC", "-ffp-contract=off", "-w", *inc, "-c", os.path.join(SRC, name), "-o", objs[-1]])
+    for path in (os.path.join(SRC, "wbvh_build.cpp"), os.path.join(SRC, "sheen_table.cpp"),
+                 os.path.join(HERE, "fake_hip", "fake_hip.cpp")):
+        objs.append(str(out / (os.path.basename(path) + ".o")))
+        jobs.append(["g++", "-std=c++17", "-O1", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", *inc, "-c", path, "-o", objs[-1]])
+    for p in [subprocess.Popen(j) for j in jobs]:
+        assert p.wait() == 0
+    so = str(out / "libplugin_on_fake_hip.so")
+    subprocess.run(["g++", "-shared", "-Wl,-Bsymbolic", "-Wl,--allow-multiple-definition", *objs, "-o", so, "-lpthread"], check=True)
+    return so
+
+
+@pytest.fixture(scope="module")
+def fake(lib):
+    p = pa.Plugin(lib)
+    f = p.lib
+    for name in ("fake_pending", "fake_live", "fake_mallocs", "fake_launches", "fake_null_counters"):
+        getattr(f, name).restype = C.c_long
+    f.fake_fail_malloc.argtypes = [C.c_long]
+    f.fake_fail_launch.argtypes = [C.c_char_p, C.c_long]
+    assert len(p.devices()) == 1
+    return p
+
+
+@pytest.fixture
+def plugin(fake):
+    fake.lib.fake_rounds(3)
+    fake.lib.fake_lazy(0)
+    yield fake
+    fake.lib.fake_lazy(0)
+    fake.lib.fake_fail_malloc(0)
+    fake.lib.fake_fail_launch(b"", 0)
+    fake.profile(0)
+    fake.release()
+
+
+def params(**k):
+    return pa.render_params(spp=1, first_sample=0, seed=1, max_depth=8, rr_start=3, **k)
+
+
+def test_failed_round_leaves_nothing_queued(plugin, host):
+    # The bounce loop queues a round ahead of the path count it waits for. When a launch of that round fails,
+    # its traversal is queued and will publish a count, in the word and under the tag that the next call waits for.
+    s = host.generate(1, 16, 16, 0.25)
+    plugin.render_ex(s, params())
+    plugin.lib.fake_lazy(1)
+    plugin.lib.fake_fail_launch(b"k_surface", 2)
+    with pytest.raises(RuntimeError):
+        plugin.render_ex(s, params())
+    assert plugin.lib.fake_pending() == 0
