@@ -640,6 +640,7 @@ void GuideState::Init(hipStream_t s) {
 
 void GuideState::EnsureBatch(size_t n) {
     if (cap >= n) return;
+    cap = 0;  // a failed growth leaves no capacity
     out.ensure(n * 48 * sizeof(float));
     rec.ensure(n * 6 * size_t(kGuideRecords) * sizeof(float4));
     cap = n;
@@ -647,9 +648,10 @@ void GuideState::EnsureBatch(size_t n) {
 
 void GuideState::EnsureTrain(size_t n) {
     if (trainCap >= n) return;
+    trainCap = 0;
+    ringHead = ringValid = 0;  // the ring starts over in the new buffer
     train.ensure(n * kGRec * sizeof(float));
     trainCap = n;
-    ringHead = ringValid = 0;  // the ring starts over in the new buffer
 }
 
 void GuideState::Infer(const int *queue, const int *count, int maxCount, const float4 *h0, const float4 *h1,

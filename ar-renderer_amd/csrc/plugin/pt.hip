@@ -2142,6 +2142,7 @@ __global__ __launch_bounds__(kBlock) void k_gather_tiled(SceneArg sp, Bufs b, in
 
 void EnsureBatch(PTScene &pt, size_t n) {
     if (pt.cap >= n) return;
+    pt.cap = 0;  // a failed growth leaves no capacity: some buffers are freed by then
     auto f4 = [&](DevBuf &b, size_t members) { b.ensure(n * members * sizeof(float4)); };
     f4(pt.ray, 4); f4(pt.path, 4); f4(pt.vertex, 4); f4(pt.prev, 2); f4(pt.shadow, 4); f4(pt.emit, 2);
     f4(pt.L, 1); f4(pt.xyz, 1);

@@ -77,3 +77,66 @@ def test_failed_round_leaves_nothing_queued(plugin, host):
     with pytest.raises(RuntimeError):
         plugin.render_ex(s, params())
     assert plugin.lib.fake_pending() == 0
+
+
+def grow_and_fail(plugin, small, large, call):
+    """call(small), then call(large) with its k-th allocation failing, for every k; yields after each failure."""
+    call(small)
+    k = 0
+    while True:
+        k += 1
+        before = plugin.lib.fake_mallocs()
+        plugin.lib.fake_fail_malloc(k)
+        try:
+            call(large)
+        except RuntimeError:
+            assert plugin.lib.fake_mallocs() - before == k
+            yield k
+            continue
+        plugin.lib.fake_fail_malloc(0)
+        return
+
+
+@pytest.mark.parametrize("flags", [0, pa.RENDER_GUIDE | pa.RENDER_GUIDE_TRAIN], ids=["plain", "guided"])
+def test_failed_growth_leaves_no_missing_buffer(plugin, host, flags):
+    # The batch's buffers are sized by the largest batch so far. A growth that fails half way has freed some of
+    # them: a smaller batch must not run on what is left.
+    s = host.generate(1, 16, 16, 0.25)
+
+    def call(spp):
+        plugin.render_ex(s, pa.render_params(spp=spp, first_sample=0, seed=1, max_depth=8, rr_start=3, flags=flags))
+
+    call(1)
+    whole = plugin.lib.fake_live()
+    plugin.release()
+    failures = 0
+    for _ in grow_and_fail(plugin, 1, 4, call):
+        failures += 1
+        call(1)
+        assert plugin.lib.fake_live() == whole
+        plugin.release()
+        call(1)
+    assert failures > 15
+    assert plugin.lib.fake_live() == whole
+
+
+def test_failed_growth_of_the_training_ring(plugin, host):
+    s = host.generate(1, 16, 16, 0.25)
+    flags = pa.RENDER_GUIDE | pa.RENDER_GUIDE_TRAIN
+
+    def call(replay):
+        plugin.tune_set("guide_replay", replay)
+        plugin.render_ex(s, params(flags=flags))
+
+    try:
+        plugin.tune_set("guide_batch", 256)
+        call(1 << 12)
+        whole = plugin.lib.fake_live()
+        plugin.lib.fake_fail_malloc(1)  # the ring is all that grows
+        with pytest.raises(RuntimeError):
+            call(1 << 13)
+        call(1 << 12)
+        assert plugin.lib.fake_live() == whole
+    finally:
+        plugin.tune_set("guide_batch", 1 << 18)
+        plugin.tune_set("guide_replay", 1 << 20)
