@@ -524,6 +524,7 @@ PRGPU_API int prgpu_film_reset(int deviceIndex, int width, int height) {
         if (width <= 0 || height <= 0) throw std::runtime_error("invalid film size");
         Device &d = Get(deviceIndex);
         size_t n = size_t(width) * size_t(height) * 3 * sizeof(double);
+        d.filmW = d.filmH = 0;  // no film if what follows fails
         d.filmSum.ensure(n);
         d.filmSq.ensure(n);
         PG_CHECK(hipMemsetAsync(d.filmSum.p, 0, n, d.stream));
@@ -542,7 +543,7 @@ PRGPU_API int prgpu_film_read(int deviceIndex, double *sum, double *sumsq) {
     try {
         Enumerate();
         Device &d = Get(deviceIndex);
-        if (!d.filmSum.p || !sum) return 1;
+        if (!d.filmSum.p || d.filmW <= 0 || !sum) return 1;
         size_t n = size_t(d.filmW) * size_t(d.filmH) * 3 * sizeof(double);
         PG_CHECK(hipMemcpyAsync(sum, d.filmSum.p, n, hipMemcpyDeviceToHost, d.stream));
         if (sumsq) PG_CHECK(hipMemcpyAsync(sumsq, d.filmSq.p, n, hipMemcpyDeviceToHost, d.stream));

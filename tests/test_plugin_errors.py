@@ -140,3 +140,17 @@ def test_failed_growth_of_the_training_ring(plugin, host):
     finally:
         plugin.tune_set("guide_batch", 1 << 18)
         plugin.tune_set("guide_replay", 1 << 20)
+
+
+@pytest.mark.parametrize("k", [1, 2])
+def test_failed_film_reset_leaves_no_film(plugin, host, k):
+    s = host.generate(1, 16, 16, 0.25)
+    plugin.film_reset(16, 16)
+    plugin.render_resident(s, params())
+    plugin.lib.fake_fail_malloc(k)
+    with pytest.raises(RuntimeError):
+        plugin.film_reset(32, 32)
+    with pytest.raises(RuntimeError, match="not reset"):
+        plugin.render_resident(s, params())
+    with pytest.raises(RuntimeError):
+        plugin.film_read(16, 16)
