@@ -177,8 +177,8 @@ Device &Get(int index) {
     if (index < 0 || index >= int(gDevices.size())) throw std::runtime_error("no such GPU device");
     Device &d = *gDevices[size_t(index)];
     PG_CHECK(hipSetDevice(d.id));
-    if (!d.stream) {
-        PG_CHECK(hipStreamCreateWithFlags(&d.stream, hipStreamNonBlocking));
+    if (!d.scratch) {  // the last to be set
+        if (!d.stream) PG_CHECK(hipStreamCreateWithFlags(&d.stream, hipStreamNonBlocking));
         hipDeviceProp_t prop;
         PG_CHECK(hipGetDeviceProperties(&prop, d.id));
         d.cus = prop.multiProcessorCount;
@@ -634,8 +634,9 @@ PRGPU_API int prgpu_release(int deviceIndex) {
 namespace {
 pgpu::GuideState &EnsureGuide(pgpu::Device &d) {
     if (!d.guide) {
-        d.guide = std::make_unique<pgpu::GuideState>();
-        d.guide->Init(d.stream);
+        auto g = std::make_unique<pgpu::GuideState>();
+        g->Init(d.stream);
+        d.guide = std::move(g);
     }
     return *d.guide;
 }

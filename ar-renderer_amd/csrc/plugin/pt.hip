@@ -2563,8 +2563,10 @@ void RenderExImpl(Device &dev, uint64_t geomKey, const prgpu::SceneDescEx &sd, c
     Params p = MakeParams(rp);
     if (p.guide) {
         if (!dev.guide || (rp.flags & prgpu::RenderGuideReset)) {
-            dev.guide = std::make_unique<GuideState>();
-            dev.guide->Init(dev.stream);
+            dev.guide.reset();
+            auto g = std::make_unique<GuideState>();
+            g->Init(dev.stream);
+            dev.guide = std::move(g);
         }
         dev.guide->EnsureBatch(pt.cap);  // per-path planes are indexed with the batch capacity
         dev.guide->blend = dev.tune.guideBlend;

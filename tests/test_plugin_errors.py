@@ -154,3 +154,35 @@ def test_failed_film_reset_leaves_no_film(plugin, host, k):
         plugin.render_resident(s, params())
     with pytest.raises(RuntimeError):
         plugin.film_read(16, 16)
+
+
+def test_failed_model_setup_leaves_no_model(plugin):
+    plugin.guide_params()
+    whole = plugin.lib.fake_live()
+    plugin.release()
+    k = 0
+    while True:
+        k += 1
+        plugin.lib.fake_fail_malloc(k)
+        try:
+            plugin.guide_params()
+        except RuntimeError:
+            plugin.lib.fake_fail_malloc(0)
+            plugin.guide_params()
+            assert plugin.lib.fake_live() == whole
+            plugin.release()
+            continue
+        break
+    assert k > 5
+
+
+def test_failed_device_setup_is_done_again(lib, tmp_path, host):
+    # (a copy of the library has a state of its own: no call has set its device up)
+    fresh = pa.Plugin(shutil.copy(lib, tmp_path / "fresh.so"))
+    fresh.lib.fake_fail_malloc.argtypes = [C.c_long]
+    fresh.devices()
+    s = host.generate(1, 16, 16, 0.25)
+    fresh.lib.fake_fail_malloc(1)  # the flags that every traversal reports to
+    with pytest.raises(RuntimeError):
+        fresh.render_ex(s, params())
+    fresh.render_ex(s, params())
