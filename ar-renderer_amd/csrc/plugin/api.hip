@@ -559,12 +559,13 @@ PRGPU_API int prgpu_profile(int deviceIndex, int mode) {
     try {
         Enumerate();
         Device &d = Get(deviceIndex);
-        d.profileMode = mode < 0 ? 0 : (mode > 2 ? 2 : mode);
-        if (d.profileMode >= 2 && !d.travCounters.p) {
+        mode = mode < 0 ? 0 : (mode > 2 ? 2 : mode);
+        if (mode >= 2 && !d.travCounters.p) {
             d.travCounters.ensure(8 * sizeof(unsigned long long));
             PG_CHECK(hipMemsetAsync(d.travCounters.p, 0, 8 * sizeof(unsigned long long), d.stream));
             PG_CHECK(hipStreamSynchronize(d.stream));
         }
+        d.profileMode = mode;
         return 0;
     } catch (const std::exception &) {
         return 1;

@@ -2349,7 +2349,7 @@ void TraceBatch(Device &dev, const DevScene &s, SceneArg ds, Params p, int passe
         AttachGuide(dev, b);
     }
     Timer timer(dev);
-    const bool stats = dev.profileMode >= 2;
+    const bool stats = dev.profileMode >= 2 && dev.travCounters.p;  // (prgpu_release frees the counters)
     const bool media = pt.hasMedia != 0, interfaces = pt.hasInterfaces != 0;
     unsigned long long *ctr = dev.travCounters.as<unsigned long long>();
     timer.Run(prgpu::KernCamera, n, nullptr, [&] {

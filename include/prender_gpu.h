@@ -402,7 +402,8 @@ PRGPU_API int prgpu_film_reset(int deviceIndex, int width, int height);
 PRGPU_API int prgpu_film_read(int deviceIndex, double *sumXYZ, double *sumSqXYZ);
 // Profiling: mode 0 off, 1 HIP-event timing of every kernel launch on the plugin's stream, 2 timing
 // plus traversal counters (a counting variant of the traversal kernels). read() returns the
-// totals since the last reset.
+// totals since the last reset. prgpu_release frees the counters: mode 2 then only times, until
+// prgpu_profile is called again.
 PRGPU_API int prgpu_profile(int deviceIndex, int mode);
 PRGPU_API int prgpu_profile_read(int deviceIndex, prgpu::ProfileStatsEx *out, int reset);
 // Run-time tuning (no reference counterpart): launch and batching parameters, set per device.

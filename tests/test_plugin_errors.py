@@ -186,3 +186,18 @@ def test_failed_device_setup_is_done_again(lib, tmp_path, host):
     with pytest.raises(RuntimeError):
         fresh.render_ex(s, params())
     fresh.render_ex(s, params())
+
+
+def test_counting_traversal_without_counters(plugin, host):
+    # prgpu_release frees the counters of profile mode 2, which stays on; and they may not be allocated.
+    s = host.generate(1, 16, 16, 0.25)
+    plugin.profile(2)
+    plugin.render_ex(s, params())
+    plugin.release()
+    plugin.render_ex(s, params())
+    plugin.profile(0)
+    plugin.lib.fake_fail_malloc(1)
+    with pytest.raises(RuntimeError):
+        plugin.profile(2)
+    plugin.render_ex(s, params())
+    assert plugin.lib.fake_null_counters() == 0
