@@ -33,7 +33,7 @@ PG_HD float safe_sqrt(float x) { return sqrtf(maxf(0.f, x)); }
 // safe_sqrt of 1 - a (a a float of any value): zero, or at least 2^-24. The device's sqrtf rescales
 // arguments below 2^-96 and tests for zero and infinity around the square-root instruction and the
 // two residuals that round its result; this range needs only those: 9 instructions instead of 17,
-// the same bits (test_sqrt_rounding.py).
+// the same bits (test_sqrt_device_gpu.py, every value of 1 - a; test_sqrt_rounding.py, the rounding step).
 PG_HD float sqrt_1m(float a) {
     const float x = maxf(0.f, 1 - a);
 #if __HIP_DEVICE_COMPILE__
