@@ -195,8 +195,8 @@ Box3 PrimBounds(const prgpu::Primitive &p) {
 // Device-resident path-tracing scene and batch buffers
 
 // Minimum waves per SIMD a kernel is compiled for (its register budget: 8 waves = 64 VGPRs,
-// 6 = 80, 5 = 96, 4 = 128, 3 = 168); 0 leaves the choice to the compiler. The traversal is
-// latency-bound and its LDS stacks allow 8 waves per SIMD, which 64 VGPRs reach without spilling.
+// 6 = 80, 5 = 96, 4 = 128, 3 = 168); 0 leaves the choice to the compiler. The traversal's LDS stacks
+// allow 8 waves per SIMD, which 64 VGPRs reach without spilling.
 // The plain material families take 174-190 VGPRs unconstrained (2 waves) and 168 at 3 waves without
 // spills in scenes without media; a 128-VGPR budget (4 waves) spills 26-28 registers and is slower:
 // terrain 62.2 -> 63.6 ms, cloud 17.0 -> 17.8, gems 19.3 -> 19.5. The surface stage (105-162 VGPRs)
@@ -1314,9 +1314,8 @@ __global__ __launch_bounds__(kBlock) PG_WAVES(kSurfaceWaves) void k_surface(Scen
     }
 }
 
-// Emission met by the paths of the emission queue, with its MIS weight (path.cpp:143-153,
-// 159-167): area light of the hit primitive, or the environment for an escaped path.
-// Emission met by one path of the emission queue, with its MIS weight.
+// Emission met by one path of the emission queue, with its MIS weight (path.cpp:143-153, 159-167): area
+// light of the hit primitive, or the environment for an escaped path.
 __device__ __forceinline__ void emit_vertex(const DevScene &s, const Bufs &b, int slot) {
     const int4 e = b.qe[slot];
     const int prim = e.w;
@@ -1401,7 +1400,7 @@ __device__ __forceinline__ void material_vertex(const DevScene &s, const Params 
     int mIn = int(int16_t(media & 0xffff)), mOut = int(int16_t(media >> 16));
     auto bsdf = [&] {
         if constexpr (kType == QLayered) return eval_closure(s, m, si, r.lam);
-        else return eval_surface<kType == QPlain ? -1 : kType>(s, m, si, r.lam);
+        else return eval_surface<kType == QDiffuse>(s, m, si, r.lam);
     }();
     bool alive = true;
     if constexpr (kGuided) {
@@ -2283,15 +2282,6 @@ struct Timer {
     }
 };
 
-// Traces one batch of `passes` passes (samples firstSample .. firstSample + passes - 1) to
-// completion; the per-sample results are left in the xyz / record buffers.
-
-
-// Bounce rounds per captured graph (tuning key graph_rounds; even: a replay ends on the queue it
-// started from); 0 = no graphs, the default. On configuration 2 at 1080p, replaying 4 captured
-// rounds took 27.9 ms per step against 25.4 ms for the pipelined eager loop (late, nearly empty
-// bounces still launch the whole-batch grids a graph bakes in, and a replay costs more than it
-// saves in synchronisation).
 // What a captured bounce graph bakes in: the kernel variants, grids, buffer addresses and the
 // parameters the bounce kernels read (not the sample range, seed or clamp, which only the camera
 // and finish kernels use).
@@ -2339,6 +2329,8 @@ int AwaitPublished(hipStream_t st, const unsigned long long *word, uint32_t tag)
     }
 }
 
+// Traces one batch of `passes` passes (samples firstSample .. firstSample + passes - 1) to
+// completion; the per-sample results are left in the xyz / record buffers.
 void TraceBatch(Device &dev, const DevScene &s, SceneArg ds, Params p, int passes, int npix, int sw) {
     PTScene &pt = *dev.pt;
     hipStream_t st = dev.stream;
@@ -2439,7 +2431,8 @@ void TraceBatch(Device &dev, const DevScene &s, SceneArg ds, Params p, int passe
     if (!dev.profileMode && !p.guide && graphRounds > 0) {
         // Unprofiled, unguided renders replay graphRounds captured bounces per launch (an even
         // count, so every replay starts from queue A) with grids sized for the whole batch, and
-        // read the path count back once per replay instead of once per bounce.
+        // read the path count back once per replay instead of once per bounce. Off by default: late,
+        // nearly empty bounces still launch the whole-batch grids.
         const int tgrid = TraceGrid(dev, n);
         const uint64_t key = BounceKey(p, b, ds, tgrid, shadeGrid, media, interfaces, s.emitters, pt.hasLayered) ^
                              (uint64_t(graphRounds) << 56);
@@ -2516,8 +2509,6 @@ void TraceBatch(Device &dev, const DevScene &s, SceneArg ds, Params p, int passe
     CheckTraceFlags(dev);
 }
 
-// Guided rendering trains the model after every batch: up to guideSteps Adam steps of guideBatch
-// records each (the records of the batch's paths, in the order they were written).
 // Passes per batch: bounded by the path budget (the queue capacity), so that the state fits
 // comfortably in HBM.
 int PassesPerBatch(const Device &dev, int npix, int spp) {

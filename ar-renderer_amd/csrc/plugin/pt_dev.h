@@ -1128,21 +1128,20 @@ PG_HD void dielectric_bx(const DevScene &s, const prgpu::Material &m, Lambda &la
     }
 }
 
-// kFamily: -1 = any plain material, else the material family the caller guarantees (0 diffuse,
-// 1 conductor, 2 dielectric), which removes the other families' code from the caller. The closure's
-// fields are joined in locals and written once: written through the branches, the record would stay
-// in scratch memory.
-template <int kFamily = -1>
+// A plain material's closure. kDiffuse: the caller guarantees a diffuse one (the guided launch), which
+// removes the other families' code. The closure's fields are joined in locals and written once: written
+// through the branches, the record would stay in scratch memory.
+template <bool kDiffuse = false>
 PG_HD BSDF eval_surface(const DevScene &s, const prgpu::Material &m, const Surf &si, Lambda &lam) {
     int type;
     float etaD = 1, ax = 0, ay = 0;
     SS ba, bb;
-    if (kFamily == 0 || (kFamily < 0 && m.type == prgpu::MatDiffuse)) {
+    if (kDiffuse || m.type == prgpu::MatDiffuse) {
         BxDF x;
         diffuse_bx(s, m, si, lam, x);
         type = x.type;
         ba = x.a;
-    } else if (kFamily == 1 || (kFamily < 0 && m.type == prgpu::MatConductor)) {
+    } else if (m.type == prgpu::MatConductor) {
         BxDF x;
         conductor_bx(s, m, si, lam, 0.f, x);
         type = x.type;

@@ -55,12 +55,6 @@ struct DRay {
     float ox, oy, oz, dx, dy, dz;
 };
 
-struct DHit {
-    float t;
-    int prim;  // original primitive index, -1 = miss
-    float b1, b2;
-};
-
 // Reference Moller-Trumbore, no contraction. Returns true and updates t/b1/b2 on a closer hit.
 __device__ __forceinline__ bool dev_hit_triangle(const DRay &r, float p0x, float p0y, float p0z, float e1x, float e1y,
                                                  float e1z, float e2x, float e2y, float e2z, float tMax, float *tOut,
@@ -428,8 +422,10 @@ __device__ __forceinline__ int feed_take(RayFeed &f, int *counter, FeedLds *fl, 
 // The loop of a persistent traversal, run by whole blocks. begin(i, r, t) loads item i's ray into r
 // and starts t; end(i, r, t) takes a finished query's result and may start the item's next query,
 // returning true. Finished lanes call end when the wave next takes rays, so that neither interrupts
-// the others' steps. Every step completes a node or a record of at least one lane, and a query
-// visits each of them at most once, so the loop ends.
+// the others' steps. Every step completes a node or a record of at least one lane. A node is visited at
+// most once by a query (references lead down the tree only) and adds at most eight references, of which
+// one from a slot without a child, which only extreme distances enter (see wbvh.h), is to a record; so a
+// query takes a bounded number of steps and the loop ends.
 template <bool kStats, class Begin, class End>
 __device__ __forceinline__ void trace_queue(const TraceCtx &c, int n, int *counter, uint32_t *lds, int tid, TraceStats *st,
                                             Begin begin, End end) {

@@ -1,5 +1,10 @@
 // 8-wide quantised BVH for the MI355X traversal kernels.
 //
+// The node follows the published compressed wide BVH (Ylitie, Karras, Laine, "Efficient Incoherent Ray
+// Traversal on GPUs Through Compressed Wide BVHs", HPG 2017): a local grid of 8-bit planes, and children
+// addressed by two bases and a byte each. The byte's meaning and the order of traversal are this file's
+// and trace_dev.h's own.
+//
 // Layout in HBM:
 //   WNode[]  80 bytes of node in a 128-byte line. Child boxes are quantised to 8 bits per axis
 //            against the node's origin and power-of-two scale, rounded outwards so every decoded

@@ -1,7 +1,7 @@
 """spec_sample (pt_dev.h) evaluates a spectrum at four wavelengths with one switch and one search in
 step; spec_eval evaluates one. Compiled for the host, both must return the same bits for every kind
-that a scene can hold: constant, sigmoid, blackbody, Sellmeier, Cauchy, the 95-sample table, and
-piecewise tables of 0 to 130 knots, at wavelengths below, on, between and above the knots.
+that a scene can hold: constant, sigmoid, blackbody, Sellmeier, Cauchy, the 95-sample table, an image
+texture (which has no value by itself: zero), and piecewise tables of 0 to 130 knots, at wavelengths below, on, between and above the knots.
 """
 import os
 import shutil
@@ -44,6 +44,7 @@ int main() {
         std::memcpy(q->p, bk7, sizeof bk7);
         q = add(prgpu::SpecCauchy, 0, scale);
         q->p[0] = 1.5f; q->p[1] = 4200;
+        add(prgpu::SpecImage, 0, scale);
         add(prgpu::SpecTable95, prgpu::kSpectrumSamples, scale);
         for (int i = 0; i < prgpu::kSpectrumSamples; ++i) knots.push_back(u(g));
         for (int n : sizes) {
