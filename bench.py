@@ -30,8 +30,9 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, os.path.join(ROOT, "ar-renderer_amd"))
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
-# HBM bytes per launch of the dominant kernel, from rocprofv3 FETCH_SIZE / WRITE_SIZE counter runs
-# scaled by a copy kernel of known size; written by hand from the committed summary.
+# HBM bytes per launch of the traversal, from rocprofv3 FETCH_SIZE / WRITE_SIZE counter runs scaled by a
+# copy kernel of known size, and its VALU issue and lane counters; written by hand from the runs. They are
+# of the kernels as they were then: a change to the traversal takes new runs.
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "trace_bounce_terrain_1080p_traffic.md")
 METRIC = "Msamples/s and equal-time relMSE, guided vs plain PT, 1080p on one MI355X"
 
@@ -513,14 +514,17 @@ def main():
             avg_ms = kernels[dominant]["ms"] / max(1, kernels[dominant]["launches"])
             # `frac` prices the algorithmic bytes (every node and record fetch counted as if it came
             # from HBM) against the HBM peak; `frac_hbm_traffic` prices the counter-measured HBM bytes
-            # of one launch. Most node and record re-reads hit L2 / MALL, and the SIMDs' issue slots are
-            # full (counters: VALU busy, 58 % of lanes active), so HBM bandwidth is not the limit.
-            roofline = {"bound": "hbm", "kernel": dominant, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
-                        "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+            # of one launch. Most node and record re-reads hit L2 / MALL. What bounds the traversal is VALU
+            # issue: the counters of the same file find the SIMDs' issue slots full.
+            trav_bound = dominant == "intersect" and traffic is not None
+            roofline = {"bound": "valu" if trav_bound else "hbm", "kernel": dominant, "achieved": round(achieved, 1),
+                        "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+                        "frac_of": "HBM peak, every fetch priced as if from HBM",
                         "traffic": traffic,
                         "frac_hbm_traffic": (round(traffic / (avg_ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)
                                              if traffic else None),
-                        "limited_by": "VALU issue at 58 % of lanes active; nodes and records come from L2 / MALL",
+                        "limited_by": ("VALU issue (slots full, 58 % of lanes active in the counter run); nodes and "
+                                       "records come from L2 / MALL" if trav_bound else None),
                         "algorithmic_bytes_per_item": round(per, 1),
                         "items_per_launch": round(kernels[dominant]["items"] / max(1, kernels[dominant]["launches"]), 1),
                         "avg_launch_ms": round(kernels[dominant]["ms"] / max(1, kernels[dominant]["launches"]), 4)}
